@@ -3,19 +3,17 @@
 //
 // Pipeline of one build (all on the caller's stream, one host sync in the Python layer
 // to size the outputs, none inside this file):
-//   1. tile_flags / tile_fill      Morton (SFC) rank of every 4x4x4 tile of bins
-//   2. bin_atoms                   fractional coords -> floor (wrap), bin, SFC key, and
-//                                  an atomic slot inside the key's bin
-//   3. scan                        bin starts (counting sort == single-digit radix sort)
-//   4. scatter_atoms               atom id -> sorted slot
-//   5. finish_bins                 stable order inside each bin, then the SoA cell list
-//                                  (fp32 position relative to the bin origin + id,
-//                                  packed floor) in SFC order
-//   6. search<false>               per-target degree (one workgroup per tile, region of
-//                                  (T+2P)^3 bins staged in LDS, one lane per target)
+//   1. tile_rank                   Morton (SFC) rank of every tile of bins
+//   2. bin_atoms                   fractional coords -> floor (wrap), bin, SFC key, and the
+//                                  atom's cell-list record
+//   3-5. tile_hist, tile_scatter, tile_sort   counting sort into the cell list: fp32 position
+//                                  relative to the bin origin + id, packed floor, in SFC order
+//   6. search<0>                   per-target degree and row words (one workgroup per tile,
+//                                  region of (T+2P)^3 bins staged in LDS, one lane per target),
+//                                  and the tile's region map
 //   7. scan                        per-tile edge offsets in SFC tile order
-//   8. search<true>                edges: lanes stage (src, shift) records in LDS, the
-//                                  workgroup then streams them out with coalesced stores
+//   8. expand, search<1>           edges: row words decoded into LDS, then streamed out with
+//                                  16-byte stores; the few tiles the count flagged swept again
 //
 // Reference stages replaced (dynamis_state/src/csrc/graph/radius_graph_kernels.cu):
 // wrap :596-605, selective images :18-141 (here: periodic bin wrap, no image atoms),
@@ -64,7 +62,6 @@ dg_status fail(dg_status st, const std::string& msg)
 
 constexpr int kRegPerThread = (kMaxRegion + kBlock - 1) / kBlock;
 constexpr int kBinSortMax = 128;
-constexpr int kExpandIlp = 4;  // 64-edge steps per iteration of the expansion (even)
 
 // Whether a device-wide flag word still reads 0 (a device-scope load, so a flag another
 // XCD set is seen): raising flags only then keeps the atomics on one address few.
@@ -74,9 +71,9 @@ __device__ __forceinline__ bool flag_clear(int64_t* w)
 }
 
 // search_kernel<1> work of a tile, set by the count pass
-constexpr int kFixOver = 1;     // a target has more than K neighbours
-constexpr int kFixChunked = 2;  // the region needs more than two LDS chunks (or no slots)
-constexpr int kFix2 = 4;        // the region needs two LDS chunks (slots hold both)
+constexpr int kFixOver = 1;     // a target has more row words than its list holds
+constexpr int kFixChunked = 2;  // no row words: the region needs more than two LDS chunks, the
+                                // region map is full, or the count recorded none
 #ifndef DG_FIXGRID
 #define DG_FIXGRID 512
 #endif
@@ -127,12 +124,13 @@ __device__ __forceinline__ float bin_xkey(const float4& e, const XKey& k)
 // Also clears the bin counts (bcnt) for the binning that follows.
 __global__ void tile_rank_kernel(GridArgs g, int64_t ntiles, int* __restrict__ tile_of_rank,
                                  int* __restrict__ rank_of_tile, int* __restrict__ bcnt,
-                                 int64_t nbins, int64_t* __restrict__ totals)
+                                 int64_t nbins, int64_t* __restrict__ totals, int64_t* __restrict__ tbase)
 {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     if (blockIdx.x == 0 && threadIdx.x < 8) totals[threadIdx.x] = 0;  // the build's totals and flags
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < nbins; q += stride) bcnt[q] = 0;
     for (int64_t lin = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; lin < ntiles; lin += stride) {
+        tbase[lin] = 0;  // (the cursors of the region map lie there until the tiles are counted)
         const int X[3] = {(int)(lin % g.ntl[0]), (int)((lin / g.ntl[0]) % g.ntl[1]),
                           (int)(lin / ((int64_t)g.ntl[0] * g.ntl[1]))};
         int f[3] = {0, 0, 0};
@@ -642,7 +640,6 @@ __global__ void finish_targets_kernel(int64_t nbins, int64_t n, const int* __res
 
 // ---------------------------------------------------------------- neighbour search
 struct SearchArgs {
-    int64_t align_max_edges;  // line-aligned wave ranges in the expansion up to this edge total
     double C[9];
     double Cinv[9];
     double hC[9];  // bin step vectors: row d = C[d] / nb[d]
@@ -655,9 +652,14 @@ struct SearchArgs {
     float inv_hax, inv_hby, inv_hcz;  // reciprocals of the diagonal bin steps
     int nb[3], P[3], T[3], ntl[3], R[3], pbc[3];
     int tb, nregion;
+    float inv_R0, inv_R01, inv_T[3];  // 1 / R0, 1 / (R0 R1), 1 / T (small_div)
+    int wrap1;  // a region bin lies at most one cell outside the grid on every periodic axis
     int64_t ntiles;
     float toff, hi_off;  // d2' = d2 - toff: edge iff bits(d2') < lo_bits, band iff d2' <= hi_off
     uint32_t lo_bits;
+    // the count pass's bounds on d2'' = d2 - mid (mid = fl(r^2)): edge iff d2'' < 0 unless
+    // |d2''| <= band or d2'' <= low, which the exact test settles
+    float mid, band, low;
     const float4* spos;
     const uint32_t* sflr;
     const int* sid;    // atom id of every cell-list entry
@@ -694,12 +696,28 @@ struct SearchArgs {
     int64_t capacity;
     int64_t* totals;
     const int64_t* out_ids;  // written for atom i: out_ids[i] (null: i); positions use i
-    // Per-target neighbour slots (K region indices each), or null.  Entries go in groups
-    // of 8 (16 bytes), group-major: group g of target j at slot + 8 * (g * nslot + j), so
-    // the groups that neighbouring targets fill at about the same time share cache lines.
-    uint16_t* slot;
-    int K;
-    int64_t nslot;  // targets (group row length)
+    const int* wid;  // the id written for cell-list entry g (sid, or out_ids of it)
+    // Row words (null: none recorded).  A target's edges are kept as one 32-bit word per stencil
+    // row that holds any: the region index of the row's last candidate (12 bits) above the
+    // row's edge mask (20 bits, bit i: candidate last - i); a longer row takes two words, the
+    // first candidates first.  Words go in groups of four (16 bytes), group-major: group g of
+    // target j at words + 4 * (g * nrow + j), so that the groups that neighbouring targets fill
+    // at about the same time share cache lines.  nw[j]: words of target j (kWordsOver: its list
+    // was too short, and search_kernel<1> writes its edges).
+    uint32_t* words;
+    uint8_t* nw;
+    int Kw;          // words a target's list holds (a multiple of 4)
+    int64_t nrow;    // targets (group row length)
+    // The region map: for each tile, from entry tmap[tile].x on, one pair per region entry (its
+    // cell-list index, packed image shift of its bin - floor of its atom).  Tiles take their
+    // part of the map in the order in which they finish, from one of npools pools of equal size
+    // (cursors in the tile offsets' place, which are written after the count, one 128-byte line
+    // each; taken from a single cursor, 4860 tiles' atomics alone took 0.37 ms); what a part
+    // holds is the same whatever the order.
+    int2* map;
+    int64_t mapcap;
+    int npools;
+    int2* tmap;  // (its first entry, its entries)
     int xsplit;     // bins ordered by x unless *xflag (see tile_sort_kernel): quarter-bin row ends
 };
 
@@ -712,6 +730,16 @@ __device__ __forceinline__ bool masked_targets(const SearchArgs& a)
 __device__ __forceinline__ bool listed_targets(const SearchArgs& a)
 {
     return a.subset && !masked_targets(a);
+}
+
+// The kernel's arguments (a SearchArgs by value, the first parameter) read again from the
+// kernarg segment, behind an opaque pointer: what a cold part of the search needs is then loaded
+// there, instead of being held in scalar registers (and spilled) across the sweep.
+__device__ __forceinline__ const SearchArgs& kernarg_search()
+{
+    auto p = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const SearchArgs*)(const char*)p;
 }
 
 // Output order -> tile rank.  Consecutive workgroups go round-robin to the 8 XCDs; the
@@ -731,97 +759,37 @@ __device__ __forceinline__ int64_t xcd_tile_rank(int64_t b, int64_t ntiles)
 }
 
 // LDS of one search workgroup.
-//   qbuf   the staged region: float4 (position relative to the tile origin, atom id) per
-//          entry while distances are tested; reused as ExpandStage by the expansion;
-//   rt/bt  region bin table (rp: first entry of each region bin, rg: its cell-list start)
-//          while the region is staged; reused as the batch tables of the expansion.
-// The count pass adds the per-lane slot staging (lb) and still fits four workgroups per
-// CU; the fix-up write pass adds the per-entry shift table T.
-constexpr int kStage = 64 * kExpandIlp;  // edges one wave stages per step
-// Edges whose outputs span whole 128-byte lines from a line-aligned start: 32 edges are 256
-// bytes of int64 ids, 384 of fp32 shifts (and of fp32 vectors), 128 of fp32 distances.
-constexpr int kLineEdges = 32;
-// Line-aligned wave ranges pay while the slot array plus a small share of the outputs stay
-// under a budget, and cost time past it (a rule fitted to measurements on this part: at
-// C3 the write stage takes 0.545 ms aligned against 0.645 ms; with 448 MB of slots, or with
-// C3's edge vectors, aligned ranges are 4-10 % slower).
-constexpr double kAlignBudget = 564e6;      // bytes
-constexpr double kAlignOutShare = 0.065;    // of the output bytes
-static_assert(kLineEdges <= 64 * kExpandIlp, "a wave's head is fetched in one step");
-// CAP: region entries staged (one LDS chunk, or two for the dense tiles of expand2)
-// STG: edges a wave stages per step (64 per unit of the expansion's ILP)
-template <int CAP, int STG = kStage>
-struct ExpandStageT {
-    int2 e[CAP + 1];  // per region entry: source atom id, packed (bin shift - floor)
-    int st_src[kBlock / 64][STG];
-    int st_dst[kBlock / 64][STG];
-    uint32_t st_S[kBlock / 64][STG];
-};
-typedef ExpandStageT<kCap> ExpandStage;
-struct BatchTab {
-    int off[kBlock + 1];  // edge offsets of the batch's targets
-    int tid[kBlock];
-    uint32_t tf[kBlock];
-};
-constexpr int kQBytes = (int)sizeof(float4) * (kCap + 1);
-static_assert(sizeof(ExpandStage) <= (size_t)kQBytes, "expansion view exceeds the region buffer");
+//   qbuf   the staged region: position relative to the tile centre per entry (the fix-up pass:
+//          and the atom id), with room behind it for the candidates read past a row's end;
+//   rt     region bin table: the byte offset of each region bin's first entry, as 32-bit words
+//          (rp) or, with quarter-bin row ends, as four 16-bit words per bin (rq): its quarters'.
+// Positions alone (12 bytes an entry) let the count pass fit five workgroups per CU; the fix-up
+// write pass adds the per-entry shift table T.
+constexpr int kWordBits = 20;                 // candidates in a row word's mask
+constexpr int kCountWaves = 5;                // waves per SIMD of the count pass
+constexpr int kWordsOver = 255;               // nw of a target whose list was too short
+constexpr int kRowMax = 28;                   // candidates of a row swept at a time (one mask register)
+static_assert(2 * kCap <= 1 << (32 - kWordBits), "a region index fits the row word");
 
-constexpr int kRing = 16;  // slot entries a lane stages in LDS (two groups of 8)
-
-// Byte address of ring entry k2 / 2 (mod 16) of the lane whose ring starts at byte lane_off
-// (a multiple of 32): lane_off | (k2 & 30) in one VALU op (the compiler emits an and and an
-// add for it).
-__device__ __forceinline__ uint32_t ring_at(int k2, uint32_t lane_off)
-{
-    uint32_t r;
-    asm("v_and_or_b32 %0, %1, 30, %2" : "=v"(r) : "v"(k2), "v"(lane_off));
-    return r;
-}
+template <int ENT>
 struct SearchLds {
-    __align__(16) unsigned char qbuf[kQBytes];
-    int tbs[kTileMax * kTileMax * kTileMax + 1];  // bin starts of the tile
+    static constexpr int kEnt = ENT;  // bytes of a region entry
+    __align__(16) unsigned char qbuf[ENT * (kCap + 3)];
+    union {
+        int tbs[kTileMax * kTileMax * kTileMax + 1];  // bin starts of the tile, while a batch's targets
+                                                      // are looked up
+        __align__(16) uint32_t ring[kBlock][4];       // (count) then per-lane groups of row words
+    };
+    uint32_t rt[2 * kMaxRegion + 2];
     int64_t w64[kBlock / 64];
     int w32[kBlock / 64];
     int64_t bc[2];  // workgroup broadcasts
 };
-struct CountLds : SearchLds {
-    int rp[kMaxRegion + 1];                     // first region entry of each region bin
-    __align__(16) uint16_t lb[kBlock][kRing];   // per-lane ring of slot entries
-};
-struct FixLds : SearchLds {
-    int rp[kMaxRegion + 1];
+struct CountLds : SearchLds<12> {};
+struct FixLds : SearchLds<16> {
     uint32_t T[kCap + 1];  // packed (bin image shift - source floor) per entry
 };
-struct ExpandLds : SearchLds {
-    BatchTab bt;
-};
-// The expansion of two-chunk tiles: the same members, a region buffer for 2 kCap entries.
-struct Expand2Lds {
-    __align__(16) unsigned char qbuf[sizeof(ExpandStageT<2 * kCap>)];
-    int tbs[kTileMax * kTileMax * kTileMax + 1];
-    int64_t w64[kBlock / 64];
-    int w32[kBlock / 64];
-    int64_t bc[2];
-    BatchTab bt;
-};
-template <int CAP> struct ExpandLdsOf { typedef ExpandLds type; };
-template <> struct ExpandLdsOf<2 * kCap> { typedef Expand2Lds type; };
-// Per wave, the edge vectors and distances of one step (STG edges) as the bytes they take
-// in the outputs (v: 3 per edge, d: 1 per edge), so 16-byte chunks go out as they are.
-template <typename VT, int STG>
-struct VecStageT {
-    __align__(16) VT v[kBlock / 64][3 * STG];
-    __align__(16) VT d[kBlock / 64][STG];
-};
-// The expansion with edge vectors / distances of type VT, in steps of 64 * kVecIlp edges.
-// (Half the steps -- 8 KB less staging, four workgroups per CU for fp32 vectors -- measured
-// slower: C3 1.27 vs 1.21 ms.)
-constexpr int kVecIlp = kExpandIlp;
-template <typename VT>
-struct ExpandVLds : ExpandLds {
-    VecStageT<VT, 64 * kVecIlp> vs;
-};
-static_assert(sizeof(CountLds) <= 40960, "count pass must fit four workgroups per CU");
+static_assert(sizeof(CountLds) <= 32000, "count pass must fit five workgroups per CU (LDS goes in 1280 bytes)");
 template <int MODE>
 struct LdsOf { typedef CountLds type; };
 template <>
@@ -893,28 +861,52 @@ __device__ __forceinline__ void emit_edge(const SearchArgs& a, int64_t o, int sr
 }
 
 // ---------------------------------------------------------------- region bins
+// x / y for 0 <= x < 2^16 and 1 <= y < 2^11, inv = fl(1 / y): the quotient is at least 1 / (2 y)
+// from the next integer, far more than its rounding (an integer division by a run-time divisor
+// takes about twenty instructions, and staging a region takes eight of them per bin).
+__device__ __forceinline__ int small_div(int x, float inv) { return (int)(((float)x + 0.5f) * inv); }
+
+// Coordinates of region bin rb inside the region.
+__device__ __forceinline__ void region_coords(const SearchArgs& a, int rb, int* r)
+{
+    r[2] = small_div(rb, a.inv_R01);
+    const int q = rb - r[2] * (a.R[0] * a.R[1]);
+    r[1] = small_div(q, a.inv_R0);
+    r[0] = q - r[1] * a.R[0];
+}
+
+// Grid bin w and periodic image sb of region bin r (region_coords) of the tile at bin g0; false
+// outside the grid on a non-periodic axis (an empty bin).
+__device__ __forceinline__ bool region_wrap(const SearchArgs& a, const int* g0, const int* r, int* w, int* sb)
+{
+    bool ok = true;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int gg = g0[d] - a.P[d] + r[d], nb = a.nb[d];
+        int q = 0;
+        if (a.pbc[d]) {
+            if (a.wrap1)
+                q = gg < 0 ? -1 : (gg >= nb ? 1 : 0);
+            else
+                q = floor_div(gg, nb);
+        } else {
+            ok = ok && gg >= 0 && gg < nb;
+        }
+        sb[d] = q;
+        w[d] = gg - q * nb;
+    }
+    return ok;
+}
+
 // Bin-list key of region bin rb of the tile at bin g0 (periodic wrap on pbc axes); false
 // outside the grid on a non-periodic axis (an empty bin).
 __device__ __forceinline__ bool region_bin_key(const SearchArgs& a, const int* g0, int rb,
                                                int64_t* key)
 {
-    const int R0 = a.R[0], R1 = a.R[1];
-    const int r[3] = {rb % R0, (rb / R0) % R1, rb / (R0 * R1)};
-    int w[3];
-    bool ok = true;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const int gg = g0[d] - a.P[d] + r[d];
-        if (a.pbc[d]) {
-            const int m = gg % a.nb[d];
-            w[d] = m < 0 ? m + a.nb[d] : m;
-        } else {
-            ok = ok && gg >= 0 && gg < a.nb[d];
-            w[d] = gg;
-        }
-    }
-    if (!ok) return false;
-    const int t0 = w[0] / a.T[0], t1 = w[1] / a.T[1], t2 = w[2] / a.T[2];
+    int r[3], w[3], sb[3];
+    region_coords(a, rb, r);
+    if (!region_wrap(a, g0, r, w, sb)) return false;
+    const int t0 = small_div(w[0], a.inv_T[0]), t1 = small_div(w[1], a.inv_T[1]), t2 = small_div(w[2], a.inv_T[2]);
     const int l0 = w[0] - t0 * a.T[0], l1 = w[1] - t1 * a.T[1], l2 = w[2] - t2 * a.T[2];
     const int tl = t0 + a.ntl[0] * (t1 + a.ntl[1] * t2);
     *key = (int64_t)a.rank_of_tile[tl] * a.tb + (l0 + a.T[0] * (l1 + a.T[1] * l2));
@@ -953,368 +945,502 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------- edge expansion
-// Stages the tile's region into ExpandStage::e as (source atom id, packed bin shift -
-// floor) pairs -- 8 bytes per entry -- bin by bin from the cell list.  The caller has
-// finished every use of the float4 view of the region buffer.
-// GIDX: an entry names its source by cell-list index instead of atom id; MAP: by the id
-// written for it (a.out_ids), for expansions that need no positions.
-template <int CAP, bool GIDX = false, bool MAP = false>
-__device__ __forceinline__ void stage_pairs(const SearchArgs& a, typename ExpandLdsOf<CAP>::type& sh,
-                                            const int* g0)
-{
-    ExpandStageT<CAP>& X = *(ExpandStageT<CAP>*)sh.qbuf;
-    {
-        int rcnt[kRegPerThread], rst[kRegPerThread];
-        const int mysum = region_bins(a, g0, rcnt, rst);
-        int total;
-        int ex = block_excl_scan<int, kBlock>(mysum, sh.w32, &total);
-        const int R0 = a.R[0], R1 = a.R[1];
-#pragma unroll
-        for (int h = 0; h < kRegPerThread; ++h) {
-            const int rb = kRegPerThread * threadIdx.x + h;
-            if (rcnt[h] > 0) {
-                const int r[3] = {rb % R0, (rb / R0) % R1, rb / (R0 * R1)};
-                int sb[3];
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    const int gg = g0[d] - a.P[d] + r[d];
-                    sb[d] = a.pbc[d] ? floor_div(gg, a.nb[d]) : 0;
-                }
-                for (int i = 0; i < rcnt[h]; ++i) {
-                    const int gidx = rst[h] + i;
-                    const uint32_t fl = a.sflr[gidx];
-                    const int src = GIDX ? gidx : (MAP ? out_id(a, a.sid[gidx]) : a.sid[gidx]);
-                    X.e[ex + i] = make_int2(src, (int)pack3(sb[0] - unpack3(fl, 0),
-                                                                     sb[1] - unpack3(fl, 1),
-                                                                     sb[2] - unpack3(fl, 2)));
-                }
-            }
-            ex += rcnt[h];
-        }
-        if (threadIdx.x == 0) X.e[CAP] = make_int2(0, 0);
-    }
+// The edges of a tile are written by a few workgroups (parts), each a range of its outputs that
+// starts on a 128-byte line (32 edges are 256 bytes of ids, 384 of shifts), in blocks of kSub
+// edges: the row words of the block's targets are decoded into LDS, one entry per edge, and the
+// edges then go out in 16-byte stores that fill whole lines.  The targets' ids may lie off the
+// sources' lines (row 1 of a [2, E] array): a block then writes those of the edges `skew` further
+// on.
+//
+// Bound by the stores: 1M atoms (90.5M edges, 2.53 GB) in 0.50-0.515 ms, against 0.595 ms with
+// one workgroup per tile and the target ids off their lines; a probe that only stores the same
+// pattern takes 0.46 ms with every line whole and 0.53 ms with the ids 80 bytes off.  Plain
+// stores instead of non-temporal ones take 0.63 ms, and the same kernel without the next
+// block's words fetched ahead (its loads then wait for the stores before them) 0.67 ms.
+constexpr int kLine = 32;                       // edges whose outputs span whole lines
+constexpr int kSub = 1024;                      // edges of a block
+constexpr int kWaveEdges = kSub / (kBlock / 64);
+constexpr int kSkewMax = 16;                    // 8-byte ids of a line
+// A part's setup (region pairs, target tables) costs about as much as a block: parts grow with
+// the tiles' number, to whole tiles in large boxes (1M atoms: 0.67 ms at two blocks a part, 0.55
+// at four, 0.50-0.515 at eight to sixteen; 100k atoms: 0.067 ms at two, 0.088 at one).
+constexpr double kPartBlocks = 10;              // blocks of a part, at most
+constexpr double kPartsWanted = 4096;           // parts that fill the chip for a few rounds
 
+template <typename VT, bool GROUPS>
+struct ExpandLds {
+    // per edge of the block: target in the batch and region entry (kNoEdge: the edge is written
+    // by search_kernel<1>); then its packed shift
+    uint32_t ent[kSub + kSkewMax];
+    __align__(16) uint32_t shift[kSub + 2];
+    // the region's pairs: id to write, packed shift (where there are no vectors)
+    int2 pair[GROUPS && std::is_void<VT>::value ? kCap : 1];
+    // the batch's targets: first edge and first row word (with the batch's totals behind them),
+    // id to write, floor, cell-list index (vectors)
+    int off[kBlock + 1];
+    int woff[kBlock + 1];
+    int tid[kBlock];
+    uint32_t tf[kBlock];
+    int tg[std::is_void<VT>::value ? 1 : kBlock];
+    int t01[2][2];  // the first and last target of a block and of the next
+    int2 s2[kBlock / 64];
+    int w32[kBlock / 64];
+    // edge vectors and distances as the bytes they take in the outputs
+    __align__(16) typename std::conditional<std::is_void<VT>::value, int, VT>::type
+        v[std::is_void<VT>::value ? 4 : 3 * kSub],
+        d[std::is_void<VT>::value ? 4 : kSub];
+};
+constexpr int kPoolLine = 16;  // 64-bit words between the region map's cursors
+// waves per SIMD of the expansion (fp64 vectors: three by their LDS)
+template <typename VT>
+constexpr int expand_waves = std::is_same<VT, double>::value ? 3 : 5;
+constexpr uint32_t kNoEdge = 0xFFFFFFFFu;
+constexpr uint32_t kZero3 = (uint32_t)kFloorBias * 0x00100401u;  // pack3(0, 0, 0)
+
+// Part s of S of tile ord for workgroup b: the parts of a tile go to one XCD (the dispatch deals
+// consecutive workgroups to the 8 XCDs in turn), so that they share its region map and words.
+__device__ __forceinline__ void part_of(int64_t b, int64_t ntiles, int S, int64_t* ord, int* s)
+{
+    const int64_t grp = b / (8 * S);
+    const int r = (int)(b - grp * (8 * S));
+    const int m = (int)min<int64_t>(8, ntiles - 8 * grp);
+    *s = r / m;
+    *ord = 8 * grp + (r - *s * m);
 }
 
-// Writes edge k < K of every target of the tile from its slot (region entries staged by
-// stage_pairs; ebase = output offset of the tile's first edge).  Each batch of up to 256
-// targets has its edges split evenly over the waves; a wave walks its range 64 edges at a
-// time, lane e finding its target by a short forward walk from the wave's current target.
-// Edges k >= K are left to search_kernel<1>.
-// PLAIN: edges go out in 16-byte groups staged in LDS; with VT (float or double) the edge
-// vectors and distances too, staged in *vsp (a VecStageT<VT>); without PLAIN every edge is
-// written by its lane (emit_edge, vectors included).
-template <bool PLAIN, int CAP, typename VT = void, int ILP = kExpandIlp>
-__device__ __forceinline__ void expand_tile(const SearchArgs& a, typename ExpandLdsOf<CAP>::type& sh,
-                                            int tbeg, int ntg, int64_t ebase, void* vsp = nullptr)
+// Two neighbouring row words of a lane, on their way from memory.
+struct WordPair {
+    uint32_t w[2];
+    int t[2];  // their targets in the batch (the second's, or the first's again)
+    int live;  // how many there are
+};
+
+// Writes part s of S of the edges of tile ord (of the target ids, those skew further on), from
+// the row words of its targets and its region map.
+// GROUPS: the edges go out in 16-byte groups, with VT (float or double) the edge vectors and
+// distances too; otherwise every edge is written by its lane (emit_edge).
+template <typename VT, bool GROUPS>
+__device__ __forceinline__ void expand_part(const SearchArgs& a, ExpandLds<VT, GROUPS>& sh, int64_t ord, int s, int S,
+                                            int skew)
 {
-    static_assert(ILP % 2 == 0, "two edges per 16-byte chunk of sources / targets");
-    constexpr int kStg = 64 * ILP;  // edges a wave stages per step
-    ExpandStageT<CAP, kStg>& X = *(ExpandStageT<CAP, kStg>*)sh.qbuf;
-    BatchTab& B = sh.bt;
-    const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
-    const int NWv = kBlock / 64;
-    constexpr bool plain = PLAIN;
     constexpr bool kVec = !std::is_void<VT>::value;
-    static_assert(PLAIN || !kVec, "the per-lane path writes vectors itself");
+    constexpr bool kStaged = GROUPS && !kVec;
     typedef typename std::conditional<kVec, VT, float>::type VTn;  // (a type when VT is void)
-    for (int k0 = 0; k0 < ntg; k0 += kBlock) {
-        const int nbatch = min(kBlock, ntg - k0);
-        const int j = tbeg + k0 + threadIdx.x;
-        const bool active = (int)threadIdx.x < nbatch;
-        const int mycnt = active ? a.cnt[j] : 0;
-        int btot;
-        const int ex = block_excl_scan<int, kBlock>(mycnt, sh.w32, &btot);
-        if (active) {
-            const int sidx = listed_targets(a) ? a.tsidx[j] : j;
-            B.off[threadIdx.x] = ex;
-            // (the plain path writes B.tid as it is: the id to write; with vectors it also
-            // indexes the target's position, and the id is mapped when staged)
-            B.tid[threadIdx.x] = (plain && !kVec) ? out_id(a, a.sid[sidx]) : a.sid[sidx];
-            B.tf[threadIdx.x] = a.sflr[sidx];
-        }
-        if (threadIdx.x == 0) B.off[nbatch] = btot;
-        __syncthreads();  // region entries and the batch tables visible to all waves
-
-        // the waves' ranges split at output offsets that are multiples of line: with
-        // kLineEdges the 16-byte groups of every full step fill whole 128-byte lines of each
-        // output (the edge total, from the count stage, decides: see kAlignBudget)
-        const int line = a.totals[0] <= a.align_max_edges ? kLineEdges : 4;
-        auto split = [&](int ww) {
-            if (ww == 0) return 0;
-            if (ww == NWv) return btot;
-            const int64_t g = ebase + ((int64_t)btot * ww) / NWv;
-            const int64_t al = (g + line - 1) & ~(int64_t)(line - 1);
-            return (int)min<int64_t>(al - ebase, btot);
-        };
-        const int E0 = split(w), E1 = split(w + 1);
-        int tcur = 0;
-        {
-            int lo = 0, hi = nbatch;  // target containing E0
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (B.off[mid] <= E0) lo = mid; else hi = mid;
-            }
-            tcur = rfl(lo);
-        }
-        const int64_t wbase = ebase + E0;
-        const char* __restrict__ sl = (const char*)a.slot + (size_t)16 * (tbeg + k0);
-        const uint64_t gstep = 16ull * (uint64_t)a.nslot;  // bytes between a target's groups
-
-        // Edges [b0, b1) of the batch (b1 - b0 <= 64 * ILP), lane-strided: edge
-        // b0 + 64u + lane -> source id, target id, packed shift; ok = false past b1 or for
-        // k >= K (left to search_kernel<1>).  All slot loads are issued before the first
-        // entry is looked up.  Advances tcur to the target of edge b1 - 1.
-        // Two halves: locate() finds (target, k) of edges [b0, b1) and issues their slot
-        // loads -- unconditionally (edges past b1 or with k >= K load a valid dummy), so all
-        // ILP loads are in flight together -- and advances tcur to the target of
-        // edge b1 - 1; resolve() turns them into (source id, target id, packed shift).  The
-        // plain path locates the next step before storing this one, so the wait on its
-        // loads does not also wait on the stores (the memory counter is shared).
-        struct Loc {
-            int tt[ILP], kk[ILP], raw[ILP];
-        };
-        auto locate = [&](int b0, int b1, Loc& L) {
-            int t = tcur;
-#pragma unroll
-            for (int u = 0; u < ILP; ++u) {
-                const int e = b0 + 64 * u + lane;
-                L.kk[u] = a.K;
-                L.tt[u] = t;
-                if (e < b1) {
-                    while (B.off[t + 1] <= e) ++t;
-                    L.tt[u] = t;
-                    L.kk[u] = e - B.off[t];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < ILP; ++u) {
-                const uint64_t at = L.kk[u] < a.K ? (uint64_t)(uint32_t)(L.kk[u] >> 3) * gstep +
-                                                        (16u * (uint32_t)L.tt[u] + 2u * (L.kk[u] & 7))
-                                                  : 0ull;
-                L.raw[u] = (int)*(const uint16_t*)(sl + at);
-            }
-            // the lane holding edge b1 - 1 has its target in t
-            if (b1 > b0) tcur = __builtin_amdgcn_readlane(t, (b1 - 1 - b0) & 63);
-        };
-        // with vectors, region entries name their source by cell-list index (rg), which
-        // also indexes the positions in cell-list order
-        int rg[ILP];
-        auto resolve = [&](const Loc& L, int* rs, int* rd, uint32_t* rS, bool* rok) {
-#pragma unroll
-            for (int u = 0; u < ILP; ++u) {
-                rok[u] = L.kk[u] < a.K;
-                const int2 en = X.e[rok[u] ? min(L.raw[u] >> 4, CAP) : CAP];
-                const uint32_t ft = B.tf[L.tt[u]];
-                if constexpr (kVec) {
-                    rg[u] = en.x;
-                    rs[u] = a.sid[en.x];
-                } else {
-                    rs[u] = en.x;
-                }
-                rd[u] = B.tid[L.tt[u]];
-                rS[u] = pack3(unpack3((uint32_t)en.y, 0) + unpack3(ft, 0),
-                              unpack3((uint32_t)en.y, 1) + unpack3(ft, 1),
-                              unpack3((uint32_t)en.y, 2) + unpack3(ft, 2));
-            }
-        };
-        auto fetch = [&](int b0, int b1, int* rs, int* rd, uint32_t* rS, bool* rok) {
-            Loc L;
-            locate(b0, b1, L);
-            resolve(L, rs, rd, rS, rok);
-        };
-        // per-lane stores of the fetched edges (ranges not aligned to 4 edges, and the
-        // vector / distance outputs)
-        auto store_lanes = [&](int b0, const int* rs, const int* rd, const uint32_t* rS,
-                               const bool* rok) {
-#pragma unroll
-            for (int u = 0; u < ILP; ++u) {
-                if (!rok[u]) continue;
-                const int64_t o = wbase + (b0 + 64 * u + lane - E0);
-                const int S0 = unpack3(rS[u], 0), S1 = unpack3(rS[u], 1), S2 = unpack3(rS[u], 2);
-                if constexpr (plain && !kVec) {
-                    __builtin_nontemporal_store((int64_t)rs[u], a.out_src + o);
-                    __builtin_nontemporal_store((int64_t)rd[u], a.out_dst + o);
-                    const v3f sv = {(float)S0, (float)S1, (float)S2};
-                    __builtin_nontemporal_store(sv, (v3f*)(a.out_shift + 3 * o));
-                } else {
-                    emit_edge(a, o, rs[u], rd[u], S0, S1, S2);
-                }
-            }
-        };
-
-        int rs[ILP], rd[ILP];
-        uint32_t rS[ILP];
-        bool rok[ILP];
-        if constexpr (!plain) {
-            for (int b0 = E0; b0 < E1; b0 += 64 * ILP) {
-                fetch(b0, min(E1, b0 + 64 * ILP), rs, rd, rS, rok);
-                store_lanes(b0, rs, rd, rS, rok);
-            }
-        } else {
-            // Groups of 4 edges that start at a multiple of 4 in the output are staged in
-            // LDS and written as 16-byte stores: 2 for the 4 sources, 2 for the targets, 3
-            // for the shifts, every one 16-byte aligned.  The edges before the first line
-            // boundary (up to kLineEdges - 1, only at the start of a batch) and the up-to-3
-            // after the last group are stored per lane, so no 16-byte store of this wave
-            // touches another wave's edges.  A slot left to search_kernel<1> (k >= K)
-            // receives a placeholder here and its edge there, later on the same stream.
-            const int head = min((int)((line - (wbase & (line - 1))) & (line - 1)), E1 - E0);
-            const int A0 = E0 + head;
-            const int A1 = A0 + ((E1 - A0) & ~3);
-            if (head > 0) {
-                fetch(E0, A0, rs, rd, rS, rok);
-                store_lanes(E0, rs, rd, rS, rok);
-            }
-            int* st_s = X.st_src[w];
-            int* st_d = X.st_dst[w];
-            uint32_t* st_S = X.st_S[w];
-            // with vectors: this lane's edges' canonical vectors and distances (fp64, as
-            // emit_edge computes them), and the wave's staging rows for them
-            VTn rv[ILP][3], rdd[ILP];
-            VTn* st_v = nullptr;
-            VTn* st_dd = nullptr;
-            if constexpr (kVec) {
-                VecStageT<VTn, kStg>& VS = *(VecStageT<VTn, kStg>*)vsp;
-                st_v = VS.v[w];
-                st_dd = VS.d[w];
-            }
-            auto vectors = [&]() {
-                if constexpr (kVec) {
-#pragma unroll
-                    for (int u = 0; u < ILP; ++u) {
-                        double ps[3], pt[3], vv[3];
-                        load_pos(a.cpos, a.f64, rg[u], ps);  // (cell-list order: local)
-                        load_pos(a.pos, a.f64, rd[u], pt);
-                        const double dd = canon_d2(ps, pt, unpack3(rS[u], 0), unpack3(rS[u], 1),
-                                                   unpack3(rS[u], 2), a.C, vv);
-                        rv[u][0] = (VTn)vv[0];
-                        rv[u][1] = (VTn)vv[1];
-                        rv[u][2] = (VTn)vv[2];
-                        rdd[u] = (VTn)sqrt(dd);
-                    }
-                }
-            };
-            // Full steps of 64 * ILP edges run branch-free: the next step's slot loads
-            // are issued before this step's stores and consumed right behind them, in
-            // straight-line code, so the wait on the loads leaves the stores in flight (the
-            // memory counter is shared by loads and stores).  The last, partial step is
-            // masked.
-            constexpr int kStep = 64 * ILP;
-            const int nfull = (A1 - A0) / kStep;
-            auto stage = [&](int n) {
-#pragma unroll
-                for (int u = 0; u < ILP; ++u) {
-                    const int i = 64 * u + lane;
-                    if (i < n) {
-                        if constexpr (kVec) {
-                            st_s[i] = out_id(a, rs[u]);
-                            st_d[i] = out_id(a, rd[u]);
-                        } else {
-                            st_s[i] = rs[u];
-                            st_d[i] = rd[u];
-                        }
-                        st_S[i] = rS[u];
-                        if constexpr (kVec) {
-                            st_v[3 * i] = rv[u][0];
-                            st_v[3 * i + 1] = rv[u][1];
-                            st_v[3 * i + 2] = rv[u][2];
-                            st_dd[i] = rdd[u];
-                        }
-                    }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            };
-            // 16-byte stores of n staged edges (n a multiple of 4) starting at output gb
-            auto store_groups = [&](int64_t gb, int n, auto full) {
-                const int G = n >> 2;
-                v4i* __restrict__ os = (v4i*)(a.out_src + gb);
-                v4i* __restrict__ od = (v4i*)(a.out_dst + gb);
-                v4f* __restrict__ of = (v4f*)(a.out_shift + 3 * gb);
-                // chunks of a full step: kStg / 2 of sources (and of targets), 3 kStg / 4
-                // of shifts; a loop over them masks the chunks past its count
-                constexpr int kChE = kStg / 2, kChS = 3 * kStg / 4;
-#pragma unroll
-                for (int h = 0; h < (kChE + 63) / 64; ++h) {
-                    const int c = 64 * h + lane;  // 16-byte chunk: edges 2c, 2c + 1
-                    if (c < (full ? kChE : 2 * G)) {
-                        const v4i vs = {st_s[2 * c], 0, st_s[2 * c + 1], 0};
-                        const v4i vd = {st_d[2 * c], 0, st_d[2 * c + 1], 0};
-                        __builtin_nontemporal_store(vs, os + c);
-                        __builtin_nontemporal_store(vd, od + c);
-                    }
-                }
-#pragma unroll
-                for (int h = 0; h < (kChS + 63) / 64; ++h) {
-                    const int c = 64 * h + lane;  // 16-byte chunk: shift floats 4c .. 4c + 3
-                    if (c < (full ? kChS : 3 * G)) {
-                        float f[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int fi = 4 * c + i;
-                            f[i] = (float)unpack3(st_S[fi / 3], fi % 3);
-                        }
-                        const v4f vf = {f[0], f[1], f[2], f[3]};
-                        __builtin_nontemporal_store(vf, of + c);
-                    }
-                }
-                if constexpr (kVec) {
-                    // the staged rows are the outputs' bytes: n edges are 3 n VT of vector
-                    // and n VT of distance, whole 16-byte chunks (n is a multiple of 4)
-                    constexpr int kPer = 16 / (int)sizeof(VTn);  // VT per chunk
-                    constexpr int kChV = 3 * kStg / kPer, kChD = kStg / kPer;
-                    if (a.out_vec) {
-                        v4i* __restrict__ ov = (v4i*)((VTn*)a.out_vec + 3 * gb);
-                        const v4i* sv = (const v4i*)st_v;
-#pragma unroll
-                        for (int h = 0; h < (kChV + 63) / 64; ++h) {
-                            const int c = 64 * h + lane;
-                            if (c < (full ? kChV : 3 * n / kPer)) __builtin_nontemporal_store(sv[c], ov + c);
-                        }
-                    }
-                    if (a.out_dist) {
-                        v4i* __restrict__ odd = (v4i*)((VTn*)a.out_dist + gb);
-                        const v4i* sd = (const v4i*)st_dd;
-#pragma unroll
-                        for (int h = 0; h < (kChD + 63) / 64; ++h) {
-                            const int c = 64 * h + lane;
-                            if (c < (full ? kChD : n / kPer)) __builtin_nontemporal_store(sd[c], odd + c);
-                        }
-                    }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            };
-            if (A0 < A1) {
-                fetch(A0, min(A1, A0 + kStep), rs, rd, rS, rok);
-                vectors();
-            }
-            for (int s0 = 0; s0 < nfull; ++s0) {
-                const int b0 = A0 + s0 * kStep;
-                stage(kStep);
-                Loc L;
-                locate(b0 + kStep, min(A1, b0 + 2 * kStep), L);  // empty past A1: dummy loads
-                store_groups(wbase + (b0 - E0), kStep, std::true_type());
-                resolve(L, rs, rd, rS, rok);
-                vectors();
-            }
-            if (nfull * kStep < A1 - A0) {
-                const int b0 = A0 + nfull * kStep;
-                stage(A1 - b0);
-                store_groups(wbase + (b0 - E0), A1 - b0, std::false_type());
-            }
-            if (A1 < E1) {
-                fetch(A1, E1, rs, rd, rS, rok);
-                store_lanes(A1, rs, rd, rS, rok);
-            }
-        }
-        ebase += btot;
-        __syncthreads();  // before the next batch rewrites the tables
+    const int tt = a.ttot[ord];
+    if (tt == 0) return;
+    const int64_t tb = a.tbase[ord];
+    if (tb + tt > a.capacity) {
+        if (threadIdx.x == 0 && !(__hip_atomic_load(&a.totals[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & kStatusCapacity))
+            atomicOr((unsigned long long*)&a.totals[1], (unsigned long long)kStatusCapacity);
+        return;
     }
+    const int fix = a.tfix[ord];
+    if (fix & kFixChunked) return;  // written by search_kernel<1>
+    // the part's outputs [p0, p1), and where the last ones of its target ids end
+    // (a part that would start at or before the tile is empty, but for one, the tile's first)
+    auto cut = [&](int q) {
+        const int64_t g = (tb + (int64_t)tt * q / S) & ~(int64_t)(kLine - 1);
+        return q == S ? tb + tt : (g <= tb ? tb & ~(int64_t)(kLine - 1) : g);
+    };
+    const int64_t r0 = cut(s), p1 = cut(s + 1), p0 = max(tb, r0);
+    if (p0 >= p1) return;
+    const int64_t q1 = min(tb + tt, p1 + skew);
+    const bool listed = listed_targets(a);
+    const int64_t kb = xcd_tile_rank(ord, a.ntiles) * a.tb;
+    const int* const tstart = listed ? a.tbstart : a.bstart;
+    const int tbeg = tstart[kb], ntg = tstart[kb + a.tb] - tbeg;
+    const int2 tm = a.tmap[ord];
+    const int2* const __restrict__ map = a.map + tm.x;
+    const int nreg = tm.y;  // region entries
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint64_t gstep = 16ull * (uint64_t)a.nrow;  // bytes between a target's word groups
+    // The region's pairs (id to write, shift) in LDS when they fit: a block's stores then wait
+    // for no load behind them (loads and stores share one in-order counter).
+    const bool staged = kStaged && nreg <= kCap;
+    constexpr int kPer = kStaged ? (kCap + kBlock - 1) / kBlock : 1;
+    int2 pr[kPer];
+    if (staged)
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) pr[u] = map[min(tid + kBlock * u, nreg - 1)];
+
+    int64_t gb = tb;  // output of the batch's first edge
+    for (int k0 = 0; k0 < ntg && gb < q1; k0 += kBlock) {
+        const int j = min(tbeg + k0 + tid, tbeg + ntg - 1);
+        const bool in = k0 + tid < ntg;
+        const int sidx = listed ? a.tsidx[j] : j;
+        const int cnt = in ? a.cnt[j] : 0;
+        const int nw0 = in ? a.nw[j] : 0;
+        const int my_id = GROUPS ? a.wid[sidx] : a.sid[sidx];
+        const uint32_t my_f = a.sflr[sidx];
+        if (staged && k0 == 0) {
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) pr[u].x = a.wid[pr[u].x];
+        }
+        // (a target without words has one that stands for all its edges)
+        const int nw = nw0 == kWordsOver ? 1 : nw0;
+        int btot, wtot;
+        const int2 ex2 = block_excl_scan2<kBlock>(make_int2(cnt, nw), sh.s2, &btot, &wtot);
+        const int ex = ex2.x;
+        sh.off[tid] = ex;
+        sh.woff[tid] = ex2.y;
+        if (tid == 0) {
+            sh.off[kBlock] = btot;
+            sh.woff[kBlock] = wtot;
+        }
+        sh.tid[tid] = my_id;
+        sh.tf[tid] = my_f;
+        if constexpr (kVec) sh.tg[tid] = sidx;
+        if (staged && k0 == 0) {
+#pragma unroll
+            for (int u = 0; u < kPer; ++u)
+                if (tid + kBlock * u < nreg) sh.pair[tid + kBlock * u] = pr[u];
+        }
+        const int64_t g0 = gb;
+        gb += btot;
+        if (gb <= p0) {  // (uniform)
+            __syncthreads();
+            continue;
+        }
+        // the batch's edges [b0, b1) are the part's, those from b2 on for their target ids only
+        const int b0 = (int)(max(p0, g0) - g0), b1 = (int)(min(q1, gb) - g0), b2 = (int)(min(p1, gb) - g0);
+        // the edges [lo, hi) of the block at output `block` (hi: target ids included), and of its
+        // place in LDS, at, the batch's edge 0
+        auto range = [&](int64_t block, int& lo, int& hi, int& at) {
+            lo = max(b0, (int)(block - g0));
+            hi = min(b1, (int)(block + kSub + skew - g0));
+            at = (int)(g0 - block);
+        };
+        // notes the first and last target of a block, for the lanes that read sh.t01[slot] after
+        // the next barrier
+        auto mark = [&](int64_t block, int slot) {
+            int lo, hi, at;
+            range(block, lo, hi, at);
+            if (cnt > 0 && ex <= lo && ex + cnt > lo) sh.t01[slot][0] = tid;
+            if (cnt > 0 && ex < hi && ex + cnt >= hi) sh.t01[slot][1] = tid;
+        };
+        auto word_at = [&](int t, int w) {
+            return *(const uint32_t*)((const char*)a.words + 16ull * (uint64_t)(tbeg + k0 + t) +
+                                      (uint64_t)(uint32_t)(w >> 2) * gstep + 4 * (w & 3));
+        };
+        // words i and i + 1 of the batch (i = the first of the block's, + 2 tid + skip); the
+        // loads go out unconditionally
+        auto fetch = [&](int slot, int skip) {
+            const int tf = sh.t01[slot][0], tl = sh.t01[slot][1];
+            const int wend = sh.woff[tl + 1], i = sh.woff[tf] + 2 * tid + skip;
+            int t = tf, th = tl + 1;  // the target with woff[t] <= i < woff[t + 1]
+            while (th - t > 1) {
+                const int mid = (t + th) >> 1;
+                const bool up = sh.woff[mid] <= i;
+                t = up ? mid : t;
+                th = up ? th : mid;
+            }
+            WordPair P;
+            P.live = min(max(wend - i, 0), 2);
+            int t2 = t;
+            if (P.live == 2)
+                while (sh.woff[t2 + 1] <= i + 1) ++t2;
+            P.t[0] = t;
+            P.t[1] = t2;
+            P.w[0] = word_at(t, P.live > 0 ? i - sh.woff[t] : 0);
+            P.w[1] = word_at(t2, P.live > 1 ? i + 1 - sh.woff[t2] : 0);
+            return P;
+        };
+        // writes a block's entries from its words, two per lane: a word's edges start where the
+        // words before it end.  first: the batch's edge that the first of them starts at;
+        // returns where the last ends.
+        auto decode = [&](const WordPair& P, int lo, int hi, int at, int first) {
+            uint32_t bits[2];
+            int n[2];
+            const bool over_tile = (fix & kFixOver) != 0;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                bits[k] = P.live > k ? P.w[k] & ((1u << kWordBits) - 1u) : 0u;
+                n[k] = __popc(bits[k]);
+                if (__builtin_expect(over_tile, 0) && P.live > k && a.nw[tbeg + k0 + P.t[k]] == kWordsOver) {
+                    bits[k] = 0;
+                    n[k] = a.cnt[tbeg + k0 + P.t[k]];
+                }
+            }
+            int rtot;
+            int e0 = first + block_excl_scan_dpp<kBlock>(n[0] + n[1], sh.w32, &rtot);
+            if (__builtin_expect(over_tile, 0)) {  // (those edges are written by search_kernel<1>)
+                int e1 = e0;
+                for (int k = 0; k < 2; ++k) {
+                    if (bits[k] == 0)
+                        for (int e = max(e1, lo); e < min(e1 + n[k], hi); ++e) sh.ent[at + e] = kNoEdge;
+                    e1 += n[k];
+                }
+            }
+            uint32_t* const ent = sh.ent + (at + lo);
+            const uint32_t len = (uint32_t)(hi - lo);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                // the mask's bits from the first candidate on; q: entry of the candidate before
+                // the leading bit
+                uint32_t m = bits[k] << (32 - kWordBits);
+                uint32_t q = ((uint32_t)P.t[k] << 12) + (P.w[k] >> kWordBits) - (uint32_t)kWordBits;
+                uint32_t e = (uint32_t)(e0 - lo);
+                while (m != 0u) {
+                    const uint32_t c = (uint32_t)__builtin_clz(m) + 1u;
+                    q += c;
+                    m <<= c;
+                    if (e < len) ent[e] = q;
+                    ++e;
+                }
+                e0 += n[k];
+            }
+            return first + rtot;
+        };
+        auto pair_of = [&](uint32_t en) -> int2 {
+            const uint32_t k = en == kNoEdge ? 0u : en & 4095u;
+            if constexpr (kStaged) {
+                if (staged) return sh.pair[k];
+                int2 p = map[k];
+                p.x = a.wid[p.x];
+                return p;
+            } else {
+                return map[k];
+            }
+        };
+        // the shifts of this wave's edges, from LDS: 16-byte chunks, of the groups of 4 edges in
+        // [a0, a1)
+        const int wb = kWaveEdges * wave;
+        auto store_shifts = [&](int64_t block, bool full, int a0, int a1) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            v4f* const __restrict__ of = (v4f*)(a.out_shift + 3 * block);
+#pragma unroll
+            for (int h = 0; h < 3 * kWaveEdges / 256; ++h) {
+                // chunk c: shift floats 4c .. 4c + 3, fields r .. r + 3 of the six of edges e, e + 1
+                const int c = 3 * wb / 4 + 64 * h + lane;
+                const int g = c / 3, r = c - 3 * g, e = 4 * g + r;  // (4c / 3 = 4g + r for r < 3)
+                if (full || (4 * g >= a0 && 4 * g < a1)) {
+                    const uint32_t S0 = sh.shift[e], S1 = sh.shift[e + 1];
+                    const uint64_t P = ((uint64_t)S1 << 30 | S0) >> (10 * r);
+                    const v4f vf = {(float)((int)(P & 1023u) - kFloorBias),
+                                    (float)((int)((P >> 10) & 1023u) - kFloorBias),
+                                    (float)((int)((P >> 20) & 1023u) - kFloorBias),
+                                    (float)((int)((P >> 30) & 1023u) - kFloorBias)};
+                    __builtin_nontemporal_store(vf, of + c);
+                }
+            }
+        };
+        // Writes a block whose edges are all the part's: straight-line code, so that the next
+        // block's words, fetched before, are waited for without its stores.
+        auto write_full = [&](int64_t block) {
+            v4i* const __restrict__ os = (v4i*)(a.out_src + block);
+            v4i* const __restrict__ od = (v4i*)(a.out_dst + block + skew);
+            uint32_t en[kWaveEdges / 64], et[kWaveEdges / 64];
+            int2 mp[kWaveEdges / 64];
+#pragma unroll
+            for (int u = 0; u < kWaveEdges / 64; ++u) {
+                // a lane takes two neighbouring edges at a time
+                const int i = wb + 128 * (u / 2) + 2 * lane + (u & 1);
+                en[u] = sh.ent[i];
+                et[u] = sh.ent[i + skew];
+            }
+#pragma unroll
+            for (int u = 0; u < kWaveEdges / 64; ++u) mp[u] = sh.pair[en[u] & 4095u];
+#pragma unroll
+            for (int h = 0; h < kWaveEdges / 128; ++h) {
+                const int i = wb + 128 * h + 2 * lane;
+                uint32_t S3[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) S3[k] = (uint32_t)mp[2 * h + k].y + sh.tf[en[2 * h + k] >> 12] - kZero3;
+                *(uint2*)&sh.shift[i] = make_uint2(S3[0], S3[1]);
+                const v4i vs = {mp[2 * h].x, 0, mp[2 * h + 1].x, 0};
+                const v4i vd = {sh.tid[et[2 * h] >> 12], 0, sh.tid[et[2 * h + 1] >> 12], 0};
+                __builtin_nontemporal_store(vs, os + i / 2);
+                __builtin_nontemporal_store(vd, od + i / 2);
+            }
+            store_shifts(block, true, 0, 0);
+        };
+        // Any block.
+        auto write_any = [&](int64_t block, int lo, int hi, int at, int tf0) {
+            const int i0 = max(at + lo, wb), i1 = min(at + b2, wb + kWaveEdges);
+            if constexpr (!GROUPS) {
+                for (int i = i0 + lane; i < i1; i += 64) {
+                    const uint32_t en = sh.ent[i];
+                    if (en == kNoEdge) continue;
+                    const int2 mp = map[en & 4095u];
+                    const uint32_t S3 = (uint32_t)mp.y + sh.tf[en >> 12] - kZero3;
+                    emit_edge(a, block + i, a.sid[mp.x], sh.tid[en >> 12], unpack3(S3, 0), unpack3(S3, 1), unpack3(S3, 2));
+                }
+                return;
+            }
+            // the sources of two neighbouring edges are one 16-byte store, and the shifts of four
+            // are three, where the edges are all the part's: groups of 4 at multiples of 4 outputs
+            // in [a0, a1); the up-to-3 edges before and after go per lane
+            const int a0 = (i0 + 3) & ~3, a1 = i1 & ~3;
+            const bool any = i0 < i1;
+            uint32_t en[kWaveEdges / 64];
+            int2 mp[kWaveEdges / 64];
+            int src[kWaveEdges / 64];
+#pragma unroll
+            for (int u = 0; u < kWaveEdges / 64; ++u) {
+                const int i = wb + 128 * (u / 2) + 2 * lane + (u & 1);
+                en[u] = i >= i0 && i < i1 ? sh.ent[i] : kNoEdge;
+                mp[u] = pair_of(en[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < kWaveEdges / 64; ++u) src[u] = kStaged ? mp[u].x : a.wid[mp[u].x];
+            uint32_t S3[kWaveEdges / 64];
+#pragma unroll
+            for (int u = 0; u < kWaveEdges / 64; ++u) {
+                const int i = wb + 128 * (u / 2) + 2 * lane + (u & 1);
+                const uint32_t t = en[u] == kNoEdge ? (uint32_t)tf0 : en[u] >> 12;
+                // (the fields of pack3 add without carries: a shift fits 10 bits)
+                S3[u] = en[u] == kNoEdge ? kZero3 : (uint32_t)mp[u].y + sh.tf[t] - kZero3;
+                sh.shift[i] = S3[u];
+                if constexpr (kVec) {
+                    double ps[3], pt[3], vv[3];
+                    load_pos(a.cpos, a.f64, mp[u].x, ps);
+                    load_pos(a.cpos, a.f64, sh.tg[t], pt);
+                    const double dd = canon_d2(ps, pt, unpack3(S3[u], 0), unpack3(S3[u], 1), unpack3(S3[u], 2), a.C, vv);
+                    sh.v[3 * i] = (VTn)vv[0];
+                    sh.v[3 * i + 1] = (VTn)vv[1];
+                    sh.v[3 * i + 2] = (VTn)vv[2];
+                    sh.d[i] = (VTn)sqrt(dd);
+                }
+            }
+            // the target ids of the wave's edges, skew further on (at the tile's start, the first
+            // ones too)
+            {
+                const int j0 = max(at + lo, r0 <= tb && block == r0 && wave == 0 ? 0 : wb + skew);
+                const int j1 = min(at + hi, wb + kWaveEdges + skew);
+                auto target = [&](int i) {
+                    const uint32_t e = sh.ent[i];
+                    return sh.tid[e == kNoEdge ? (uint32_t)tf0 : e >> 12];
+                };
+                if (j0 == wb + skew && j1 - j0 == kWaveEdges) {
+#pragma unroll
+                    for (int h = 0; h < kWaveEdges / 128; ++h) {
+                        const int i = wb + skew + 128 * h + 2 * lane;
+                        const v4i vd = {target(i), 0, target(i + 1), 0};
+                        __builtin_nontemporal_store(vd, (v4i*)(a.out_dst + block + i));
+                    }
+                } else {
+                    for (int i = j0 + lane; i < j1; i += 64) a.out_dst[block + i] = target(i);
+                }
+            }
+            if (!any) return;
+            v4i* const __restrict__ os = (v4i*)(a.out_src + block);
+#pragma unroll
+            for (int h = 0; h < kWaveEdges / 128; ++h) {
+                const int i = wb + 128 * h + 2 * lane;
+                if (i >= a0 && i < a1) {
+                    const v4i vs = {src[2 * h], 0, src[2 * h + 1], 0};
+                    __builtin_nontemporal_store(vs, os + i / 2);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 2; ++k)
+                        if (i + k >= i0 && i + k < i1) {
+                            const int64_t o = block + i + k;
+                            const uint32_t S = S3[2 * h + k];
+                            a.out_src[o] = src[2 * h + k];
+                            *(float3*)(a.out_shift + 3 * o) =
+                                make_float3((float)unpack3(S, 0), (float)unpack3(S, 1), (float)unpack3(S, 2));
+                            if constexpr (kVec) {
+                                if (a.out_vec)
+                                    for (int c = 0; c < 3; ++c) ((VTn*)a.out_vec)[3 * o + c] = sh.v[3 * (i + k) + c];
+                                if (a.out_dist) ((VTn*)a.out_dist)[o] = sh.d[i + k];
+                            }
+                        }
+                }
+            }
+            const bool full = i1 - i0 == kWaveEdges;
+            store_shifts(block, full, a0, a1);
+            if constexpr (kVec) {
+                // the staged rows are the outputs' bytes
+                constexpr int kPer = 16 / (int)sizeof(VTn);  // VT per chunk
+                if (a.out_vec) {
+                    v4i* const __restrict__ ov = (v4i*)((VTn*)a.out_vec + 3 * block);
+#pragma unroll
+                    for (int h = 0; h < 3 * kWaveEdges / kPer / 64; ++h) {
+                        const int c = 3 * wb / kPer + 64 * h + lane;
+                        const int q = kPer * c / 12 * 4;  // of the edges q .. q + 3
+                        if (full || (q >= a0 && q < a1)) __builtin_nontemporal_store(((const v4i*)sh.v)[c], ov + c);
+                    }
+                }
+                if (a.out_dist) {
+                    v4i* const __restrict__ odd = (v4i*)((VTn*)a.out_dist + block);
+#pragma unroll
+                    for (int h = 0; h < kWaveEdges / kPer / 64; ++h) {
+                        const int c = wb / kPer + 64 * h + lane;
+                        const int q = kPer * c & ~3;
+                        if (full || (q >= a0 && q < a1)) __builtin_nontemporal_store(((const v4i*)sh.d)[c], odd + c);
+                    }
+                }
+            }
+        };
+
+        // The blocks of kSub outputs (the first may hold target ids only, those of the batch's
+        // first edges).  A block's words are fetched while the block before it is written.
+        int64_t block = r0 + (max(g0 + b0 - skew - r0, (int64_t)0) & ~(int64_t)(kSub - 1));
+        const int64_t bend = min(g0 + (int64_t)b1, p1);  // blocks start below it
+        if (block >= bend) {
+            __syncthreads();
+            continue;
+        }
+        mark(block, 0);
+        __syncthreads();
+        WordPair P = fetch(0, 0);
+        int slot = 0;
+        auto is_full = [&](int64_t b) {
+            return kStaged && staged && fix == 0 && !(r0 <= tb && b == r0) && g0 + b0 <= b && b + kSub + skew <= g0 + b1 && b + kSub <= g0 + b2;
+        };
+        auto words_in = [&](int sl) { return sh.woff[sh.t01[sl][1] + 1] - sh.woff[sh.t01[sl][0]]; };
+        while (block < bend) {
+            int lo, hi, at;
+            if constexpr (kStaged) {
+                if (is_full(block) && words_in(slot) <= 2 * kBlock) {
+                    // (the first pair is waited for here, so that the wait inside the loop is the
+                    // one behind the loop's own stores)
+                    asm volatile("" : "+v"(P.w[0]), "+v"(P.w[1]));
+                    bool again;
+                    do {
+                        range(block, lo, hi, at);
+                        decode(P, lo, hi, at, sh.off[sh.t01[slot][0]]);
+                        const int64_t next = block + kSub;
+                        const bool more = next < bend;
+                        mark(more ? next : block, slot ^ 1);
+                        __syncthreads();
+                        P = fetch(slot ^ 1, 0);
+                        write_full(block);
+                        slot ^= 1;
+                        block = next;
+                        again = more && is_full(next) && words_in(slot) <= 2 * kBlock;
+                        __syncthreads();  // before the next block's entries are written
+                    } while (again);
+                    if (block >= bend) break;
+                }
+            }
+            range(block, lo, hi, at);
+            const int tf0 = sh.t01[slot][0], nwords = words_in(slot);
+            int first = decode(P, lo, hi, at, sh.off[tf0]);
+            for (int skip = 2 * kBlock; skip < nwords; skip += 2 * kBlock)
+            {
+                const WordPair Q = fetch(slot, skip);
+                __syncthreads();  // (before the scan's sums are written again)
+                first = decode(Q, lo, hi, at, first);
+            }
+            const int64_t next = block + kSub;
+            if (next < bend) mark(next, slot ^ 1);
+            __syncthreads();
+            if (next < bend) P = fetch(slot ^ 1, 0);
+            write_any(block, lo, hi, at, tf0);
+            slot ^= 1;
+            block = next;
+            __syncthreads();  // before the next block's entries, or the next batch's tables
+        }
+    }
+}
+
+// Takes n entries of pool p of the region map; where they start in the pool.
+__device__ __forceinline__ unsigned long long map_take(const SearchArgs& a, int p, int n)
+{
+    return atomicAdd((unsigned long long*)a.tbase + kPoolLine * p, (unsigned long long)n);
 }
 
 // Neighbour search, one tile of bins per workgroup.
@@ -1324,12 +1450,11 @@ __device__ __forceinline__ void expand_tile(const SearchArgs& a, typename Expand
 // the stencil trimmed to the cutoff sphere for lower-triangular cells), so they agree on
 // every edge and on its order.
 //
-// MODE 0 (count): per-target degree, per-tile total, and -- for tiles whose region fits
-//   in one chunk -- the target's neighbours as 2-byte LDS entry byte offsets in its slot of
-//   K entries (written 16 bytes at a time through a per-lane LDS buffer).
-// MODE 1 (fix-up write, only tiles the count pass flagged): targets with more than K
-//   neighbours get their edges k >= K by a second sweep, tiles with a chunked region are
-//   swept again and written directly.  Every other edge is written by expand_kernel.
+// MODE 0 (count): per-target degree, per-tile total, and -- for tiles whose region fits two
+//   chunks -- the target's row words and the tile's region map.
+// MODE 1 (fix-up write, only tiles the count pass flagged): targets with more words than their
+//   list holds, and tiles without words, are swept again and written directly.  Every other
+//   edge is written by expand_kernel.
 // What the count of one tile leaves for the publication / expansion of its edges.
 struct TileOut {
     int64_t tt;  // edges of the tile
@@ -1346,7 +1471,10 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
                                                typename LdsOf<MODE>::type& sh, int64_t ord)
 {
     constexpr bool WRITE = MODE == 1;
-    float4* const shq = (float4*)sh.qbuf;
+    constexpr int kEnt = LdsOf<MODE>::type::kEnt;
+    char* const qb = (char*)sh.qbuf;
+    int* const rp = (int*)sh.rt;
+    uint16_t* const rq = (uint16_t*)sh.rt;
     TileOut out;
     out.tt = 0;
     out.fix = 0;
@@ -1373,7 +1501,7 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
         }
         return out;
     }
-    if (WRITE && (a.tfix[ord] & (kFixOver | kFixChunked)) == 0) return out;  // written by an expansion
+    if (WRITE && a.tfix[ord] == 0) return out;  // written by the expansion
     if (!WRITE && masked) {
         // a tile of ghosts only (atoms with ids >= ntarg) has no targets: nothing to count
         bool mine = false;
@@ -1386,8 +1514,6 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
             return out;
         }
     }
-    for (int k = threadIdx.x; k <= a.tb; k += kBlock) sh.tbs[k] = tstart[kb + k];
-
     int64_t ebase = 0;
     if (WRITE) {
         ebase = a.tbase[ord];
@@ -1401,113 +1527,143 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
     // ---- region table: (T+2P)^3 bins around the tile, periodic wrap on pbc axes
     const int R0 = a.R[0], R1 = a.R[1];
     int rcnt[kRegPerThread], rst[kRegPerThread];
-    const int mysum = region_bins(a, g0, rcnt, rst);
+    const int mysum = region_bins(kernarg_search(), g0, rcnt, rst);
     int total;
     int rex[kRegPerThread];  // first region entry of this thread's bins
     {
         int ex = block_excl_scan<int, kBlock>(mysum, sh.w32, &total);
 #pragma unroll
         for (int h = 0; h < kRegPerThread; ++h) {
-            const int rb = kRegPerThread * threadIdx.x + h;
             rex[h] = ex;
-            if (rb < a.nregion) sh.rp[rb] = ex;
             ex += rcnt[h];
         }
-        if (threadIdx.x == 0) sh.rp[a.nregion] = total;
     }
-    __syncthreads();
     const int nchunks = (total + kCap - 1) / kCap;
     // Quarter-bin row ends (QS: count pass, lower-triangular cell; a one-chunk region whose
-    // bins are ordered by bin_xkey): staging packs into each rp word, above its 20-bit first
-    // entry, the number of the bin's entries whose key lies below each of its quarter
-    // boundaries (3 x 4 bits; 15: 15 or more), and a row then starts at the quarter of its
-    // first bin that the cutoff reaches and ends after the quarter of its last.
-    // Entries cut off this way lie beyond the padded cutoff along x alone, so they are never
-    // edges: every target's edge sequence is unchanged (the fix-up pass, which sweeps whole
-    // bins, numbers edges alike).
-    static_assert(kCap < (1 << 20), "a one-chunk region's first entries fit the rp word's 20 bits");
+    // bins are ordered by bin_xkey): the bin table holds where each quarter of a bin starts,
+    // counted by the entries whose key lies below each quarter boundary while staging, and a
+    // row then starts at the quarter of its first bin that the cutoff reaches and ends after
+    // the quarter of its last.  Entries cut off this way lie beyond the padded cutoff along x
+    // alone, so they are never edges: every target's edge sequence is unchanged (the fix-up
+    // pass, which sweeps whole bins, numbers edges alike).
+    static_assert(12 * kCap < 65536, "a one-chunk region's offsets fit 16 bits");
     const bool qsplit = QS != 0 && nchunks == 1 && a.totals[4] == 0;
-    XKey xkey;
-    xkey.hbx = a.hbx; xkey.hcx = a.hcx; xkey.hcy = a.hcy; xkey.inv_hby = a.inv_hby; xkey.inv_hcz = a.inv_hcz;
-    const int rpm = qsplit ? 0xFFFFF : -1;  // first-entry bits of an rp word
-    const float qb1 = 0.25f * a.hax, qb2 = 0.5f * a.hax, qb3 = 0.75f * a.hax;
-    // slots hold up to two chunks' entries (2-byte byte offsets in the region); a larger
-    // region is written directly by search_kernel<1>
-    // (the write pass follows what the count pass recorded: a tile it flagged as chunked --
-    // a region of more than two chunks, or a count that kept no slots -- is swept again)
-    const bool slotted = nchunks <= 2 && a.slot != nullptr && !(WRITE && (a.tfix[ord] & kFixChunked));
+    if (!qsplit) {
+#pragma unroll
+        for (int h = 0; h < kRegPerThread; ++h) {
+            const int rb = kRegPerThread * threadIdx.x + h;
+            if (rb < a.nregion) rp[rb] = kEnt * rex[h];
+        }
+        if (threadIdx.x == 0) rp[a.nregion] = kEnt * total;
+    } else if (threadIdx.x == 0) {
+        rq[4 * a.nregion] = (uint16_t)(kEnt * total);
+    }
+    // byte offset of region bin rb's first entry, in the whole region
+    auto bin_first = [&](int rb) -> int { return qsplit ? (int)rq[4 * rb] : rp[rb]; };
+    // row words name up to two chunks' entries; a larger region is written directly by
+    // search_kernel<1>, which follows what the count pass recorded: a tile flagged as chunked
+    // is swept again
+    const bool slotted = WRITE ? !(a.tfix[ord] & kFixChunked) : nchunks <= 2 && a.words != nullptr;
+    unsigned long long map_at = 0;  // (count, thread 0) the tile's first region-map entry
     int loaded = -1;
 
     // packed (image shift of region bin rb - floor of cell-list entry gidx)
     auto entry_T = [&](int rb, int gidx) -> uint32_t {
         const uint32_t fl = a.sflr[gidx];
-        const int r[3] = {rb % R0, (rb / R0) % R1, rb / (R0 * R1)};
-        int sb[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const int gg = g0[d] - a.P[d] + r[d];
-            sb[d] = a.pbc[d] ? floor_div(gg, a.nb[d]) : 0;
-        }
+        int r[3], w[3], sb[3];
+        region_coords(a, rb, r);
+        region_wrap(a, g0, r, w, sb);
         return pack3(sb[0] - unpack3(fl, 0), sb[1] - unpack3(fl, 1), sb[2] - unpack3(fl, 2));
     };
-    // every thread copies the entries of its own region bins that fall in chunk c
-    auto load_chunk = [&](int c) {
+    // every thread copies the entries of its own region bins (cnt, first cell-list entry st,
+    // first region entry ex0) that fall in chunk c
+    auto copy_bins = [&](int c, const int* cnt, const int* st, const int* ex0) {
+        const SearchArgs& k = kernarg_search();
+        const float qb1 = 0.25f * k.hax, qb2 = 0.5f * k.hax, qb3 = 0.75f * k.hax;
+        XKey xkey;
+        xkey.hbx = k.hbx; xkey.hcx = k.hcx; xkey.hcy = k.hcy; xkey.inv_hby = k.inv_hby; xkey.inv_hcz = k.inv_hcz;
         const int c0 = c * kCap;
         const int c1 = min(total, c0 + kCap);
 #pragma unroll
         for (int h = 0; h < kRegPerThread; ++h) {
             const int rb = kRegPerThread * threadIdx.x + h;
-            const int b0 = max(rex[h], c0), b1 = min(rex[h] + rcnt[h], c1);
-            if (b0 >= b1) continue;
-            const int r[3] = {rb % R0, (rb / R0) % R1, rb / (R0 * R1)};
-            float o[3];
-            region_offset(a, r[0], r[1], r[2], o);
-            const int g = rst[h] - rex[h];  // cell-list index minus region index
+            const int b0 = max(ex0[h], c0), b1 = min(ex0[h] + cnt[h], c1);
             int s1 = 0, s2 = 0, s3 = 0;  // entries below the quarter boundaries
-            for (int vv = b0; vv < b1; vv += 4) {
-                float4 e[4];
+            if (b0 < b1) {
+                int r[3];
+                region_coords(k, rb, r);
+                float o[3];
+                region_offset(k, r[0], r[1], r[2], o);
+                const int g = st[h] - ex0[h];  // cell-list index minus region index
+                for (int vv = b0; vv < b1; vv += 4) {
+                    float4 e[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (vv + u < b1) e[u] = a.spos[g + vv + u];
+                    for (int u = 0; u < 4; ++u)
+                        if (vv + u < b1) e[u] = k.spos[g + vv + u];
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (vv + u < b1) {
-                        shq[vv + u - c0] = make_float4(e[u].x + o[0], e[u].y + o[1], e[u].z + o[2], e[u].w);
-                        if constexpr (WRITE) sh.T[vv + u - c0] = entry_T(rb, g + vv + u);
-                        if constexpr (QS != 0) {
-                            const float xk = QS == 1 ? e[u].x : bin_xkey(e[u], xkey);
-                            s1 += xk < qb1;
-                            s2 += xk < qb2;
-                            s3 += xk < qb3;
+                    for (int u = 0; u < 4; ++u)
+                        if (vv + u < b1) {
+                            const float x = e[u].x + o[0], y = e[u].y + o[1], z = e[u].z + o[2];
+                            if constexpr (WRITE) {
+                                ((float4*)qb)[vv + u - c0] = make_float4(x, y, z, e[u].w);
+                                sh.T[vv + u - c0] = entry_T(rb, g + vv + u);
+                            } else {
+                                float* const to = (float*)(qb + kEnt * (vv + u - c0));
+                                to[0] = x; to[1] = y; to[2] = z;
+                            }
+                            if constexpr (QS != 0) {
+                                const float xk = QS == 1 ? e[u].x : bin_xkey(e[u], xkey);
+                                s1 += xk < qb1;
+                                s2 += xk < qb2;
+                                s3 += xk < qb3;
+                            }
                         }
-                    }
+                }
             }
-            if (QS != 0 && qsplit)  // (one chunk: [b0, b1) is the whole bin)
-                sh.rp[rb] = rex[h] | (int)((uint32_t)(min(s1, 15) | (min(s2, 15) << 4) | (min(s3, 15) << 8)) << 20);
+            if (QS != 0 && qsplit && rb < k.nregion) {  // (one chunk: [b0, b1) is the whole bin)
+                const uint32_t f = (uint32_t)(kEnt * ex0[h]);
+                sh.rt[2 * rb] = f | ((f + kEnt * s1) << 16);
+                sh.rt[2 * rb + 1] = (f + kEnt * s2) | ((f + kEnt * s3) << 16);
+            }
         }
     };
     auto ensure_chunk = [&](int c) {  // uniform
         if (loaded != c) {
             __syncthreads();
-            load_chunk(c);
+            if (loaded < 0 && c == 0) {
+                copy_bins(0, rcnt, rst, rex);
+            } else {
+                // (looked up again: the bins of the first chunk need not stay in registers)
+                int cnt[kRegPerThread], st[kRegPerThread], ex0[kRegPerThread];
+                region_bins(kernarg_search(), g0, cnt, st);
+#pragma unroll
+                for (int h = 0; h < kRegPerThread; ++h)
+                    ex0[h] = cnt[h] ? bin_first(kRegPerThread * threadIdx.x + h) / kEnt : 0;
+                copy_bins(c, cnt, st, ex0);
+            }
             __syncthreads();
             loaded = c;
         }
     };
+    // the first chunk is resident before the first target is looked up
+    ensure_chunk(0);
 
     const int nrx = 2 * a.P[0] + 1, nry = 2 * a.P[1] + 1, nrz = 2 * a.P[2] + 1;
-    int64_t tile_found = 0;
+    int tile_found = 0;  // (this lane's; a tile's total is kept as an int too)
     bool over_any = false;
 
     for (int k0 = 0; k0 < ntg; k0 += kBlock) {
         const int nbatch = min(kBlock, ntg - k0);
+        for (int k = threadIdx.x; k <= a.tb; k += kBlock) sh.tbs[k] = tstart[kb + k];
+        __syncthreads();
         const int kk = k0 + threadIdx.x;
         const int j = tbeg + kk;
         const bool in_batch = (int)threadIdx.x < nbatch;
         bool active = in_batch;
 
         // ---- per-lane target state
-        int lx = 0, ly = 0, lz = 0, my_id = 0, caller = 0, v_self = -1;
+        int lx = 0, ly = 0, lz = 0, my_id = 0, caller = 0;
+        int v_self = -kEnt;  // byte offset of the target's own region entry
         uint32_t my_f = 0;
         float t0 = 0.f, t1 = 0.f, t2 = 0.f, ux = 0.f, uy = 0.f, uz = 0.f;
         if (active) {
@@ -1516,9 +1672,10 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
                 const int mid = (lo + hi) >> 1;
                 if (sh.tbs[mid] <= j) lo = mid; else hi = mid;
             }
-            lx = lo % a.T[0];
-            ly = (lo / a.T[0]) % a.T[1];
-            lz = lo / (a.T[0] * a.T[1]);
+            const int q = small_div(lo, a.inv_T[0]);
+            lz = small_div(q, a.inv_T[1]);
+            ly = q - lz * a.T[1];
+            lx = lo - q * a.T[0];
             const int sidx = listed ? a.tsidx[j] : j;
             const float4 e = a.spos[sidx];
             my_f = a.sflr[sidx];
@@ -1527,13 +1684,14 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
             active = !masked || my_id < a.ntarg;  // (masked: a ghost atom's lane idles)
             ux = e.x; uy = e.y; uz = e.z;  // position inside its own bin
             float o[3];
-            region_offset(a, lx + a.P[0], ly + a.P[1], lz + a.P[2], o);
+            region_offset(kernarg_search(), lx + a.P[0], ly + a.P[1], lz + a.P[2], o);
             t0 = e.x + o[0]; t1 = e.y + o[1]; t2 = e.z + o[2];
             // the target's own region entry (same atom, zero shift) is never an edge
             const int rb_self = ((lz + a.P[2]) * R1 + (ly + a.P[1])) * R0 + (lx + a.P[0]);
             const int bin_start = listed ? a.bstart[kb + lo] : sh.tbs[lo];
-            v_self = (sh.rp[rb_self] & rpm) + (sidx - bin_start);
+            v_self = bin_first(rb_self) + kEnt * (sidx - bin_start);
         }
+        __syncthreads();  // (tbs is read; its place is the ring's)
         const int fx = unpack3(my_f, 0), fy = unpack3(my_f, 1), fz = unpack3(my_f, 2);
         // the target's position inside its bin in bin units (lower-triangular cells)
         // (reciprocals and the hardware square root below: their few-ulp errors are far
@@ -1543,28 +1701,16 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
         const float Oxp = Ox + (float)a.P[0];  // (orthorhombic rows: x bins from the region's first)
         const float Oxp4 = 4.f * Oxp, inv_hax4 = 4.f * a.inv_hax;  // in quarter bins (exact scalings)
 
-        // Sweep this lane's target over the resident chunk c, in the fixed order (dz, dy,
-        // x, atom) -- ascending region index; on_cand(v, edge, k) receives every candidate's
-        // byte offset in the chunk (16 x its chunk-local region index), whether it is an
-        // edge, and twice the running neighbour
-        // number, k2 = 2 k (k: the edge's number when it is one); on_step(k2) follows every
-        // step of two candidates, on_row(k2) every row.
-        //
-        // Rows are swept with one row of lookahead: the wave stays on row r until every
-        // lane has finished its row r, and a lane that finishes early goes on into its row
-        // r + 1 meanwhile, so a wave waits for its longest row less often.
-        int found2 = 0;  // twice the neighbours found so far
         // (QS 1: rprune2 - gz^2 of the layer oz = gz_oz, kept while the rows of one z
         // layer go by; gz_oz is uniform)
         float gzz = 0.f;
         int gz_oz = -1;
-        // candidate range [va, vb) of row ri (oz * nry + oy) of this lane, chunk-local;
+        const int rb_lane = (lz * R1 + ly) * R0 + lx;  // the first bin of the lane's first row
+        // candidate range of row (oz, oy) of this lane, as chunk-local byte offsets;
         // empty when the padded cutoff sphere misses the row
-        auto row_range = [&](int ri, int c0, int c1, int& va, int& vb) {
-            const int oz = ri / nry, oy = ri - oz * nry;
+        auto row_range = [&](int oz, int oy, int c0, int c1) -> int2 {
             int xlo = 0, xhi = nrx - 1;
-            int qlo = 0, qhi = 3;  // first and last quarter of the end bins
-            va = vb = 0;
+            int ql = 0, qh = 0;  // first and last quarter, in the row's quarters
             if (QS == 1 || (QS == 0 && a.lowtri == 2)) {
                 // orthorhombic: the row's bins span y in [py, py + 1] hby and z in
                 // [pz, pz + 1] hcz around the target; their gaps (less the margin) bound the
@@ -1585,23 +1731,16 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
                     const float gz = fmaxf(fmaxf(fmaf(pz, a.hcz, -a.pmargin), fmaf(-pz, a.hcz, a.gz_off)), 0.f);
                     rem2 = fmaf(-gz, gz, fmaf(-gy, gy, a.rprune2));
                 }
-                if (rem2 < 0.f) return;
+                if (rem2 < 0.f) return make_int2(0, 0);
                 const float rem = __builtin_amdgcn_sqrtf(rem2);
                 if constexpr (QS == 1) {
                     // (4 floor(u) + quarter = floor(4 u): the bins are those of floor(u))
-                    const int QL = max((int)floorf(fmaf(-rem, inv_hax4, Oxp4)), 0);
-                    const int QH = min((int)floorf(fmaf(rem, inv_hax4, Oxp4)), 4 * nrx - 1);
-                    xlo = QL >> 2;
-                    xhi = QH >> 2;
-                    if (xlo > xhi) return;
-                    if (qsplit) {
-                        qlo = QL & 3;
-                        qhi = QH & 3;
-                    }
+                    ql = max((int)floorf(fmaf(-rem, inv_hax4, Oxp4)), 0);
+                    qh = min((int)floorf(fmaf(rem, inv_hax4, Oxp4)), 4 * nrx - 1);
                 } else {
                     xlo = max((int)floorf(fmaf(-rem, a.inv_hax, Oxp)), 0);
                     xhi = min((int)floorf(fmaf(rem, a.inv_hax, Oxp)), nrx - 1);
-                    if (xlo > xhi) return;
+                    if (xlo > xhi) return make_int2(0, 0);
                 }
             } else if (QS == 2 || (QS == 0 && a.lowtri)) {
                 // bounding box of the row (bins py, pz relative to the target's bin, all x)
@@ -1617,7 +1756,7 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
                 gy = fmaxf(gy - a.pmargin, 0.f);
                 gz = fmaxf(gz - a.pmargin, 0.f);
                 const float rem2 = a.rprune2 - gy * gy - gz * gz;
-                if (rem2 < 0.f) return;
+                if (rem2 < 0.f) return make_int2(0, 0);
                 const float rem = __builtin_amdgcn_sqrtf(rem2);
                 const float sl = fminf(py * a.hbx, (py + 1.f) * a.hbx) + fminf(pz * a.hcx, (pz + 1.f) * a.hcx);
                 const float sh = fmaxf(py * a.hbx, (py + 1.f) * a.hbx) + fmaxf(pz * a.hcx, (pz + 1.f) * a.hcx);
@@ -1626,213 +1765,259 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
                     // whose a fraction is below u - xlo lies at least rem below the target
                     // in x (its shear is at most sh), one of the last bin at or above
                     // w - xhi at least rem above it (its shear is at least sl)
-                    const int QL = max((int)floorf(4.f * (Ox + (-rem - sh) * a.inv_hax)) + 4 * a.P[0], 0);
-                    const int QH = min((int)floorf(4.f * (Ox + (rem - sl) * a.inv_hax)) + 4 * a.P[0], 4 * nrx - 1);
-                    xlo = QL >> 2;
-                    xhi = QH >> 2;
-                    if (xlo > xhi) return;
-                    if (qsplit) {
-                        qlo = QL & 3;
-                        qhi = QH & 3;
-                    }
+                    ql = max((int)floorf(4.f * (Ox + (-rem - sh) * a.inv_hax)) + 4 * a.P[0], 0);
+                    qh = min((int)floorf(4.f * (Ox + (rem - sl) * a.inv_hax)) + 4 * a.P[0], 4 * nrx - 1);
                 } else {
                     xlo = max((int)floorf(Ox + (-rem - sh) * a.inv_hax) + a.P[0], 0);
                     xhi = min((int)floorf(Ox + (rem - sl) * a.inv_hax) + a.P[0], nrx - 1);
-                    if (xlo > xhi) return;
+                    if (xlo > xhi) return make_int2(0, 0);
                 }
             }
-            const int rb = ((lz + oz) * R1 + (ly + oy)) * R0 + lx;
-            int sa, sb;
-            if (QS != 0 && qsplit) {  // (wave-uniform)
-                // (all three words read unconditionally: a select, not a branch)
-                const uint32_t wl = (uint32_t)sh.rp[rb + xlo], wh = (uint32_t)sh.rp[rb + xhi],
-                               we = (uint32_t)sh.rp[rb + xhi + 1];
-                sa = (int)(wl & 0xFFFFFu) + (int)((wl >> (16 + 4 * qlo)) & (qlo ? 15u : 0u));
-                const int ch = (int)((wh >> (20 + 4 * min(qhi, 2))) & 15u);
-                sb = (int)((qhi < 3 && ch != 15 ? wh + (uint32_t)ch : we) & 0xFFFFFu);
-            } else {
-                sa = sh.rp[rb + xlo];
-                sb = sh.rp[rb + xhi + 1];
+            const int rb = rb_lane + (oz * R1 + oy) * R0;
+            if constexpr (QS != 0) {
+                if (qsplit) {  // (uniform: the region's only chunk)
+                    const int va = rq[4 * rb + ql], vb = rq[4 * rb + qh + 1];
+                    return make_int2(va, max(va, vb));
+                }
+                xlo = ql >> 2;
+                xhi = qh >> 2;
+                if (xlo > xhi) return make_int2(0, 0);
             }
-            va = max(sa, c0) - c0;
-            vb = min(sb, c1) - c0;
-            if (va >= vb) va = vb = 0;
-            va <<= 4;  // byte offsets of the 16-byte entries
-            vb <<= 4;
+            const int va = max(rp[rb + xlo] - kEnt * c0, 0), vb = min(rp[rb + xhi + 1], kEnt * c1) - kEnt * c0;
+            return va < vb ? make_int2(va, vb) : make_int2(0, 0);
         };
-        auto sweep = [&](int c, auto&& on_cand, auto&& on_step, auto&& on_row) {
-            const int c0 = c * kCap;
-            const int c1 = min(total, c0 + kCap);
-            const int vs = (v_self - c0) << 4;
-            const int nrows = nrz * nry;
-            const char* const qb = (const char*)shq;
-            // Candidates are addressed by the byte offset of their 16-byte entry in shq.
-            // [v, e): this lane's unswept part of its current row; [pv, pe): its next row,
-            // pv == pe once the lane has moved on to it (an empty or missing next row is
-            // [16, 0) until then).  A lane moves on to its next row the step it finishes its
-            // current one, so when the wave leaves row ri every lane is on its row ri + 1.
-            int v, e, pv, pe;
-            row_range(0, c0, c1, v, e);
-            if (!active) v = e = 0;
-            for (int ri = 0; ri < nrows; ++ri) {
-                pv = 0; pe = 0;
-                if (ri + 1 < nrows && active) row_range(ri + 1, c0, c1, pv, pe);
-                if (pv == pe) { pv = 16; pe = 0; }
-                if (v >= e) { v = pv; e = pe; pv = pe; }  // nothing left of row ri
-                // two candidates per step, both loads issued first (the second may be one
-                // past the range -- at most the sentinel -- and is then masked); the edge
-                // test is branch-free, the rare exact test sits behind a scalar mask test,
-                // and on_cand sees every candidate in order
-                if (__builtin_amdgcn_ballot_w64(pv != pe) != 0ull) do {
-                    const float4 q0 = *(const float4*)(qb + v), q1 = *(const float4*)(qb + v + 16);
-                    const bool in0 = v < e, in1 = v + 16 < e;
-                    // d2 - toff with the offset in the innermost fma; edge iff its bits are
-                    // below lo_bits (0 <= d2' < lo_off), band iff d2' <= hi_off
-                    float dx = q0.x - t0, dyv = q0.y - t1, dzv = q0.z - t2;
-                    const float d20 = fmaf(dzv, dzv, fmaf(dyv, dyv, fmaf(dx, dx, -a.toff)));
-                    dx = q1.x - t0; dyv = q1.y - t1; dzv = q1.z - t2;
-                    const float d21 = fmaf(dzv, dzv, fmaf(dyv, dyv, fmaf(dx, dx, -a.toff)));
-                    bool e0 = in0 & (__float_as_uint(d20) < a.lo_bits);
-                    bool e1 = in1 & (__float_as_uint(d21) < a.lo_bits);
-                    const bool b0 = in0 & !e0 & (d20 <= a.hi_off) & (v != vs);
-                    const bool b1 = in1 & !e1 & (d21 <= a.hi_off) & (v + 16 != vs);
-                    if (__builtin_expect(b0 | b1, 0)) {  // divergent: the mask test is scalar
-                        if (b0)
-                            e0 = exact_edge(a, __float_as_int(q0.w), my_id, (double)q0.x - t0,
-                                            (double)q0.y - t1, (double)q0.z - t2);
-                        if (b1)
-                            e1 = exact_edge(a, __float_as_int(q1.w), my_id, (double)q1.x - t0,
-                                            (double)q1.y - t1, (double)q1.z - t2);
-                    }
-                    // (a candidate past the range is no edge: k does not advance)
-                    on_cand(v, e0, found2);
-                    found2 += e0 ? 2 : 0;
-                    on_cand(v + 16, e1, found2);
-                    found2 += e1 ? 2 : 0;
-                    on_step(found2);
-                    // range done: from row ri on to the next row, from that one to rest (at
-                    // v = e: masked loads of entries e and e + 1, inside LDS)
-                    // (a lane already on its next row that finishes it takes [pe, pe): empty)
-                    const int nv = v + 32;
-                    const bool fin = nv >= e;
-                    v = fin ? pv : nv;
-                    e = fin ? pe : e;
-                    pv = fin ? pe : pv;
-                } while (__builtin_amdgcn_ballot_w64(pv != pe) != 0ull);
-                on_row(found2);
-            }
-        };
-        auto none = [](int) {};
-
         if constexpr (!WRITE) {
             // ---------------- count pass
-            // Slot entries are staged in a per-lane LDS ring of 16: the entry of slot k is
-            // written for every candidate (an edge keeps it: k advances), and full groups
-            // of 8 go out to the slot at the end of each row -- or within the row, before
-            // the ring could wrap onto a group not yet stored.
-            // this lane's ring: byte lane_off of sh.lb (its low five bits clear, so an entry's
-            // byte address is lane_off | (k2 & 30), one bitwise VALU)
-            static_assert(2 * kRing == 32, "ring of 16 two-byte entries per lane");
-            char* const lb0 = (char*)&sh.lb[0][0];
-            const uint32_t lane_off = threadIdx.x << 5;
-            char* const lbb = lb0 + lane_off;
             const bool slots = slotted;
-            char* const slotb = (char*)a.slot;
-            const uint64_t gstep = 16ull * (uint64_t)a.nslot;  // bytes between a target's groups
-            uint64_t goff = 16ull * (uint64_t)j;                // byte offset of group kf2 / 16
-            int kf2 = 0;                                      // 2 x entries stored (or skipped)
-            int klim = 2 * kRing - 4;                         // kf2 + 28: the in-row flush mark
-            const int K2 = 2 * a.K;
-            auto store_group = [&]() {  // the group starting at entry kf2 / 2
-                if (kf2 + 16 <= K2) *(uint4*)(slotb + goff) = *(const uint4*)(lbb + (kf2 & 16));
-                kf2 += 16;
-                klim += 16;
-                goff += gstep;
+            uint32_t* const ring = sh.ring[threadIdx.x];
+            // group g of this target's list
+            auto group = [&](int g) { return (uint4*)a.words + ((uint64_t)(uint32_t)g * (uint64_t)(uint32_t)a.nrow + (uint32_t)j); };
+            int found = 0, w = 0;  // edges, and row words recorded
+            // Records the row whose last candidate is region index last, of n candidates with
+            // the edge mask bits (bit i: candidate last - i).
+            auto put_word = [&](uint32_t word, bool put) {  // (not put: overwritten by the next)
+                ring[w & 3] = word;
+                w += put ? 1 : 0;
+                if (put && (w & 3) == 0 && w <= a.Kw) *group((w >> 2) - 1) = *(const uint4*)ring;
             };
-            auto flush = [&](int k2) {  // every full group below entry k2 / 2
-                while (kf2 + 16 <= k2) store_group();
+            auto put_row = [&](uint32_t bits, int last) {
+                found += __popc(bits);
+                if (!slots) return;
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(bits >> kWordBits != 0u) != 0ull, 0)) {
+                    put_word(((uint32_t)(last - kWordBits) << kWordBits) | (bits >> kWordBits), bits >> kWordBits != 0u);
+                    bits &= (1u << kWordBits) - 1u;
+                }
+                put_word(((uint32_t)last << kWordBits) | bits, bits != 0u);
             };
+
+            // Bound by VALU issue and, per row, by the latency of its few LDS reads: 120M VALU
+            // instructions at 1M atoms (r = 6, 90.5M edges) in 0.27 ms, against 159M in 0.345 ms
+            // for a sweep that wrote a 2-byte entry per edge (two candidates a step, 34 VALU;
+            // this one: four a step, 39), at four workgroups per CU to this one's five.
+            //
+            // Sweeps this lane's target over the resident chunk c, in the fixed order (dz, dy, x,
+            // atom) -- ascending region index.  The edge test is the sign bit of d2 - mid, shifted
+            // into a mask register, one bit per candidate and two candidates per step; a row's
+            // mask becomes its row word, so the loop holds no compare, counter or store per
+            // candidate.  The rare candidate within the band around the cutoff, or at a distance
+            // near zero, shows in two running minima: its row is then decided again, candidate
+            // by candidate, with the exact test.
+            //
+            // Rows are swept with one row of lookahead: the wave stays on row r until every
+            // lane has finished its row r, and a lane that finishes early goes on into its row
+            // r + 1 meanwhile, so a wave waits for its longest row less often.  Rows of more than
+            // kRowMax candidates go in pieces.
+            auto sweep = [&](int c) {
+                constexpr int kPieceB = kEnt * kRowMax;
+                static_assert(kRowMax % 4 == 0 && kRowMax < 32, "a piece's steps fit the mask register");
+                // (entries of a byte offset b < 65536 that is a multiple of 12: b / 12)
+                auto entries = [](int b) { return (int)(__umul24((uint32_t)b, 5462u) >> 16); };
+                const int c0 = c * kCap;
+                const int c1 = min(total, c0 + kCap);
+                const int vs = v_self - kEnt * c0;
+                const float nmid = -a.mid;
+                int oz = 0, oy = 0;    // the next row (uniform); oz = nrz: none
+                int fa = 0, fe = 0;    // what is left of the row taken last
+                bool pend = false;     // some lane has some left
+                bool center = false;   // that row is the target's own
+                // The next piece: at most kRowMax candidates of the row, and up to the target's own
+                // entry, which is skipped.
+                auto next_piece = [&]() -> int2 {
+                    if (!pend) {
+                        const int2 r = row_range(oz, oy, c0, c1);
+                        fa = r.x;
+                        fe = active ? r.y : r.x;
+                        center = oz == a.P[2] && oy == a.P[1];
+                        const bool wrap = oy + 1 == nry;
+                        oz += wrap ? 1 : 0;
+                        oy = wrap ? 0 : oy + 1;
+                    }
+                    const int pv = fa;
+                    int pe = min(fe, pv + kPieceB);
+                    fa = pe;
+                    if (center) {
+                        const bool self = vs >= pv && vs < pe;
+                        pe = self ? vs : pe;
+                        fa = self ? vs + kEnt : pe;
+                    }
+                    pend = __builtin_amdgcn_ballot_w64(fa < fe) != 0ull;
+                    return make_int2(pv, pe);
+                };
+                const int2 piece0 = next_piece();
+                int v = piece0.x, e = piece0.y;  // [v, e): this lane's unswept part of its current piece
+                int ncur = e - v, ecur = e;   // the wave's piece: its bytes, and its end
+                int2 nxt = next_piece();      // this lane's next piece
+                uint32_t M = 0;               // the masks of this lane's pieces, newest bit lowest
+                float near_hi = INFINITY, near_lo = INFINITY;  // least |d2 - mid|, least d2 - mid
+                uint64_t again = 0ull;        // lanes whose next piece is to be decided again
+                bool more = true, more2 = true;  // there is a next piece, and one after it
+                do {
+                    const int pv = nxt.x, pe = nxt.y;
+                    more = more2;
+                    // (the piece after the next is looked up before the steps, which hide its LDS
+                    // reads)
+                    more2 = more && (pend || oz < nrz);
+                    nxt = make_int2(0, 0);
+                    if (more2) nxt = next_piece();
+                    const int nnext = pe - pv;
+                    uint32_t Mp = M;              // the mask of this lane's current piece, when done
+                    const bool done = v >= e;
+                    uint64_t live = __builtin_amdgcn_ballot_w64(!done);
+                    v = done ? pv : v;
+                    e = done ? pe : e;
+                    while (live != 0ull) {
+                        if (v < e) {
+                            // four candidates per step: those past the end (at most three, inside
+                            // qbuf) leave bits that the piece's mask drops
+                            struct F3 { float x, y, z; };
+                            const F3* const q = (const F3*)(qb + v);
+                            const F3 q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
+                            auto dist = [&](const F3& p) {
+                                const float dx = p.x - t0, dy = p.y - t1, dz = p.z - t2;
+                                return fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, nmid)));
+                            };
+                            float d0 = dist(q0), d1 = dist(q1), d2 = dist(q2), d3 = dist(q3);
+                            M = __builtin_amdgcn_alignbit(M, __float_as_uint(d0), 31);
+                            M = __builtin_amdgcn_alignbit(M, __float_as_uint(d1), 31);
+                            M = __builtin_amdgcn_alignbit(M, __float_as_uint(d2), 31);
+                            M = __builtin_amdgcn_alignbit(M, __float_as_uint(d3), 31);
+                            near_hi = fminf(fminf(near_hi, fabsf(d0)), fabsf(d1));
+                            near_hi = fminf(fminf(near_hi, fabsf(d2)), fabsf(d3));
+                            near_lo = fminf(fminf(near_lo, d0), d1);
+                            near_lo = fminf(fminf(near_lo, d2), d3);
+                        }
+                        // (a lane at rest is not live, and stays at or past e)
+                        const int nv = v + 4 * kEnt;
+                        const uint64_t firstm = __builtin_amdgcn_ballot_w64(nv >= e) & live;
+                        const bool first = __builtin_amdgcn_inverse_ballot_w64(firstm);
+                        Mp = first ? M : Mp;
+                        e = first ? pe : e;
+                        v = first ? pv : nv;
+                        live &= ~firstm;
+                    }
+                    // the piece is done in every lane: its n candidates' bits, less
+                    // those swept past the end
+                    const int n = entries(ncur);
+                    uint32_t bits = (Mp >> (-n & 3)) & ((1u << n) - 1u);
+                    const uint64_t nearm = __builtin_amdgcn_ballot_w64(near_hi <= a.band) |
+                                           __builtin_amdgcn_ballot_w64(near_lo <= a.low);
+                    if (__builtin_expect((nearm | again) != 0ull, 0)) {
+                        // (what the minima saw lies in this piece or, in the lookahead, the next)
+                        if (__builtin_amdgcn_inverse_ballot_w64(nearm | again)) {
+                            bits = 0;
+                            for (int q = ecur - ncur; q < ecur; q += kEnt) {
+                                const float* const x = (const float*)(qb + q);
+                                const float dx = x[0] - t0, dy = x[1] - t1, dz = x[2] - t2;
+                                const float d = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, nmid)));
+                                bool edge = d < 0.f;
+                                if (fabsf(d) <= a.band || d <= a.low) {
+                                    // the source: its bin is the last that starts at or before it
+                                    const SearchArgs& k = kernarg_search();
+                                    const int at = q + kEnt * c0;
+                                    int lo = 0, hi = k.nregion;
+                                    while (hi - lo > 1) {
+                                        const int mid = (lo + hi) >> 1;
+                                        if (bin_first(mid) <= at) lo = mid; else hi = mid;
+                                    }
+                                    const int g = region_bin_start(k, g0, lo) + (at - bin_first(lo)) / kEnt;
+                                    edge = exact_edge(k, k.sid[g], my_id, (double)dx, (double)dy, (double)dz);
+                                }
+                                bits = (bits << 1) | (edge ? 1u : 0u);
+                            }
+                            near_hi = near_lo = INFINITY;
+                        }
+                        again = nearm;
+                    }
+                    put_row(bits, entries(ecur) - 1 + c0);
+                    ncur = nnext;
+                    ecur = pe;
+                } while (more);
+            };
+
+            const bool wave_active = __builtin_amdgcn_ballot_w64(active) != 0ull;
             for (int c = 0; c < nchunks; ++c) {
                 ensure_chunk(c);
-                if (!active) continue;
-                if (slots) {
-                    auto on_step = [&](int k2) {
-                        // k2 - kf2 <= 32 here: at most two groups to store
-                        if (k2 > klim) {
-                            store_group();
-                            if (k2 - kf2 >= 16) store_group();
-                        }
-                    };
-                    auto on_row = [&](int k2) { flush(k2); };
-                    // slot entries are byte offsets in the whole region: chunk 1's entries
-                    // follow chunk 0's kCap
-                    if (c == 0)
-                        sweep(c, [&](int v, bool, int k2) {
-                                  *(uint16_t*)(lb0 + ring_at(k2, lane_off)) = (uint16_t)v;
-                              }, on_step, on_row);
-                    else
-                        sweep(c, [&](int v, bool, int k2) {
-                                  *(uint16_t*)(lb0 + ring_at(k2, lane_off)) = (uint16_t)(v + 16 * kCap);
-                              }, on_step, on_row);
-                } else {
-                    sweep(c, [&](int, bool, int) {}, none, none);
-                }
+                if (c == 0 && k0 == 0 && slotted && threadIdx.x == 0)  // (its result is used after the sweep)
+                    map_at = map_take(a, (int)(ord % a.npools), total);
+                if (wave_active) sweep(c);
             }
-            const int found = found2 >> 1;
-            if (active) {
-                if (slots) {
-                    flush(found2);
-                    if ((found & 7) && found < a.K) *(uint4*)(slotb + goff) = *(const uint4*)(lbb + (kf2 & 16));
-                }
+            if (in_batch) {  // (inactive in the batch: masked, a ghost without edges)
                 a.cnt[j] = found;
-                if (a.counts_user) a.counts_user[caller] = found;
+                if (slots) {
+                    const bool over = w > a.Kw;
+                    if ((w & 3) && !over) *group(w >> 2) = *(const uint4*)ring;
+                    a.nw[j] = (uint8_t)(over ? kWordsOver : w);
+                    over_any = over_any || over;
+                }
+                if (active && a.counts_user) a.counts_user[caller] = found;
                 tile_found += found;
-                over_any = over_any || found > a.K;
-            } else if (in_batch) {
-                a.cnt[j] = 0;  // (masked: a ghost, no edges)
             }
             __syncthreads();
             continue;
         }
 
+        // Sweeps this lane's target over the resident chunk c, in the count pass's order;
+        // on_edge(v, k) receives every edge's byte offset in the chunk and its number.
+        int found = 0;
+        auto sweep = [&](int c, auto&& on_edge) {
+            const int c0 = c * kCap;
+            const int c1 = min(total, c0 + kCap);
+            const int vs = v_self - kEnt * c0;
+            for (int ri = 0; ri < nrz * nry; ++ri) {
+                const int2 r = row_range(ri / nry, ri % nry, c0, c1);
+                for (int v = r.x; v < r.y; v += kEnt) {
+                    const float4 q = *(const float4*)(qb + v);
+                    // d2 - toff with the offset in the innermost fma; edge iff its bits are
+                    // below lo_bits (0 <= d2' < lo_off), band iff d2' <= hi_off
+                    const float dx = q.x - t0, dy = q.y - t1, dz = q.z - t2;
+                    const float d = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, -a.toff)));
+                    bool edge = __float_as_uint(d) < a.lo_bits;
+                    if (!edge && d <= a.hi_off && v != vs)
+                        edge = exact_edge(a, __float_as_int(q.w), my_id, (double)dx, (double)dy, (double)dz);
+                    if (edge) on_edge(v, found++);
+                }
+            }
+        };
         if constexpr (WRITE) {
         // ---------------- write pass
         const int mycnt = active ? a.cnt[j] : 0;
         int btot;
         const int ex = block_excl_scan<int, kBlock>(mycnt, sh.w32, &btot);
-        if (slotted) {
-            // targets with more than K neighbours: the rest by a second sweep (over both
-            // chunks of a two-chunk region, k counting on as in the count pass)
-            const bool over = active && mycnt > a.K;
-            if (block_any<kBlock>(over, sh.w32)) {
-                const int64_t base = ebase + ex;
-                for (int c = 0; c < nchunks; ++c) {
-                    ensure_chunk(c);
-                    if (over)
-                        sweep(c, [&](int vb, bool e, int k2) {
-                            const int k = k2 >> 1, v = vb >> 4;
-                            if (e && k >= a.K && k < mycnt) {
-                                const uint32_t Tp = sh.T[v];
-                                emit_edge(a, base + k, __float_as_int(shq[v].w), my_id,
-                                          unpack3(Tp, 0) + fx, unpack3(Tp, 1) + fy, unpack3(Tp, 2) + fz);
-                            }
-                        }, none, none);
-                }
-            }
-        } else {
-            // chunked region (very dense tiles): sweep and write directly
+        // all of a tile without row words, or the targets whose list was too short
+        const bool mine = active && (!slotted || a.nw[j] == kWordsOver);
+        if (block_any<kBlock>(mine, sh.w32)) {
             const int64_t base = ebase + ex;
             for (int c = 0; c < nchunks; ++c) {
                 ensure_chunk(c);
-                if (!active) continue;
-                sweep(c, [&](int vb, bool e, int k2) {
-                    const int k = k2 >> 1, v = vb >> 4;
-                    if (e && k < mycnt) {
+                if (!mine) continue;
+                sweep(c, [&](int vb, int k) {
+                    const int v = vb / kEnt;
+                    if (k < mycnt) {
                         const uint32_t Tp = sh.T[v];
-                        emit_edge(a, base + k, __float_as_int(shq[v].w), my_id,
+                        emit_edge(a, base + k, __float_as_int(((const float4*)qb)[v].w), my_id,
                                   unpack3(Tp, 0) + fx, unpack3(Tp, 1) + fy, unpack3(Tp, 2) + fz);
                     }
-                }, none, none);
+                });
             }
         }
         ebase += btot;
@@ -1840,16 +2025,65 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
         __syncthreads();
     }
 
-    if (!WRITE) {
+    if constexpr (!WRITE) {
+        // the tile's part of the region map, bin by bin (the last sweep is done: w64, bc free)
+        bool mapped = false;
+        int64_t mb = 0;
+        if (slotted) {
+            if (threadIdx.x == 0) {
+                // (a full pool: the next ones are tried)
+                const int64_t cap = a.mapcap / a.npools;
+                int pool = (int)(ord % a.npools);
+                for (int k = 1; (int64_t)map_at + total > cap && k < a.npools; ++k) {
+                    pool = (pool + 1) % a.npools;
+                    map_at = map_take(a, pool, total);
+                }
+                sh.bc[0] = (int64_t)map_at + total <= cap ? pool * cap + (int64_t)map_at : -1;
+            }
+            __syncthreads();
+            mb = sh.bc[0];
+            mapped = mb >= 0;
+        }
+        if (mapped) {
+            // (the sweeps are done: the region's buffer holds the pairs, which then go out
+            // side by side)
+            const SearchArgs& k = kernarg_search();
+            int2* const pair = (int2*)sh.qbuf;
+            static_assert(sizeof(sh.qbuf) >= 8 * kCap, "the pairs of a chunk fit the region's buffer");
+            for (int v0 = 0; v0 < total; v0 += kCap) {
+#pragma unroll
+                for (int h = 0; h < kRegPerThread; ++h) {
+                    const int rb = kRegPerThread * threadIdx.x + h;
+                    if (rb >= k.nregion) continue;
+                    const int first = bin_first(rb) / kEnt - v0, end = bin_first(rb + 1) / kEnt - v0;
+                    if (first >= end || end <= 0 || first >= kCap) continue;
+                    int r[3], w[3], sb[3];
+                    region_coords(k, rb, r);
+                    region_wrap(k, g0, r, w, sb);
+                    // (the fields of pack3 subtract without borrows: each stays within 10 bits)
+                    const int T0 = (int)(pack3(sb[0], sb[1], sb[2]) + kZero3);
+                    for (int v = max(first, 0); v < min(end, kCap); ++v)
+                        pair[v] = make_int2(rst[h] + v - first, T0);
+                }
+                __syncthreads();
+                int2* const to = k.map + mb + v0;
+                for (int v = threadIdx.x; v < min(total - v0, kCap); v += kBlock) {
+                    const int2 p = pair[v];
+                    to[v] = make_int2(p.x, p.y - (int)k.sflr[p.x]);
+                }
+                __syncthreads();
+            }
+        }
         int64_t tt;
         block_excl_scan<int64_t, kBlock>(tile_found, sh.w64, &tt);
         const bool over = block_any<kBlock>(over_any, sh.w32);
-        const int fix = (over ? kFixOver : 0) | (slotted ? (nchunks == 2 ? kFix2 : 0) : kFixChunked);
+        const int fix = mapped ? (over ? kFixOver : 0) : kFixChunked;
         out.tt = tt;
         out.fix = fix;
-        if (MODE == 0 && threadIdx.x == 0) {
+        if (threadIdx.x == 0) {
             a.ttot[ord] = (int)tt;
             a.tfix[ord] = fix;
+            a.tmap[ord] = make_int2((int)mb, total);
             if (fix && flag_clear(&a.totals[3]))  // the fix-up pass has work
                 atomicOr((unsigned long long*)&a.totals[3], 1ull);
         }
@@ -1857,70 +2091,23 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
     return out;
 }
 
-// Writes every edge the count pass left in the slots of tile ord (output order), from a
-// region staged for up to CAP entries: kCap for most tiles (expand_kernel), 2 kCap for the
-// two-chunk tiles (inside search_kernel<1>).
-// VT: the type of the edge vectors / distances written in 16-byte groups from *vsp (void:
-// none, or written per lane).
-template <int CAP, typename VT = void>
-__device__ __forceinline__ void expand_one(const SearchArgs& a, typename ExpandLdsOf<CAP>::type& sh,
-                                           int64_t ord, void* vsp = nullptr)
-{
-    const int64_t rank = xcd_tile_rank(ord, a.ntiles);
-    const int* tstart = listed_targets(a) ? a.tbstart : a.bstart;
-    const int64_t kb = rank * a.tb;
-    const int tbeg = tstart[kb], tend = tstart[kb + a.tb];
-    const int ntg = tend - tbeg;
-    if (ntg == 0 || a.ttot[ord] == 0) return;  // (no edges: nothing to expand)
-    const int64_t ebase = a.tbase[ord];
-    if (ebase + a.ttot[ord] > a.capacity) {
-        if (threadIdx.x == 0)
-            atomicOr((unsigned long long*)&a.totals[1], (unsigned long long)kStatusCapacity);
-        return;
-    }
-    const int lin = a.tile_of_rank[rank];
-    const int g0[3] = {(lin % a.ntl[0]) * a.T[0], ((lin / a.ntl[0]) % a.ntl[1]) * a.T[1],
-                       (lin / (a.ntl[0] * a.ntl[1])) * a.T[2]};
-    // region entries: cell-list indices (grouped vectors), the ids to write (the plain
-    // path, which needs no positions), or atom indices (the per-lane path)
-    if constexpr (!std::is_void<VT>::value) {
-        stage_pairs<CAP, true>(a, sh, g0);
-        expand_tile<true, CAP, VT, kVecIlp>(a, sh, tbeg, ntg, ebase, vsp);
-    } else if (!a.out_vec && !a.out_dist) {
-        stage_pairs<CAP, false, true>(a, sh, g0);
-        expand_tile<true, CAP>(a, sh, tbeg, ntg, ebase);
-    } else {
-        stage_pairs<CAP>(a, sh, g0);
-        expand_tile<false, CAP>(a, sh, tbeg, ntg, ebase);
-    }
-}
-
-// MODE 0 (count) and MODE 1 (fix-up write): one tile per workgroup.  The fix-up also
-// expands the slots of the two-chunk tiles (their region needs the larger staging buffer).
+// MODE 0 (count) and MODE 1 (fix-up write): one tile per workgroup.
 // QS: the count with quarter-bin row ends (1: orthorhombic cells, 2: other lower-triangular
 // cells; cell list ordered by bin_xkey).
 template <int MODE, int QS = 0>
-__global__ __launch_bounds__(kBlock) void search_kernel(SearchArgs a)
+__global__ __launch_bounds__(kBlock, MODE == 0 ? kCountWaves : 1) void search_kernel(SearchArgs a)
 {
     if constexpr (MODE == 0) {
         __shared__ CountLds sh;
         search_tile<0, QS>(a, sh, blockIdx.x);
     } else {
-        __shared__ union {
-            FixLds f;
-            Expand2Lds e;
-        } u;
+        __shared__ FixLds f;
         // a grid of at most DG_FIXGRID workgroups walks the tiles: most have nothing to do,
         // and in most builds no tile has (the count pass raises totals[3] when one does)
         if (a.totals[3] == 0) return;
         for (int64_t ord = blockIdx.x; ord < a.ntiles; ord += gridDim.x) {
-            const int fix = a.tfix[ord];
-            if (fix == 0) continue;
-            if (fix & kFix2) {
-                expand_one<2 * kCap>(a, u.e, ord);
-                __syncthreads();
-            }
-            search_tile<1>(a, u.f, ord);
+            if (a.tfix[ord] == 0) continue;
+            search_tile<1>(a, f, ord);
             __syncthreads();  // before the next tile reuses the LDS
         }
     }
@@ -1930,9 +2117,6 @@ __global__ __launch_bounds__(kBlock) void search_kernel(SearchArgs a)
 // the count kernel's launcher, compiled in dg_count.hip
 void launch_count_kernel(const SearchArgs& a, unsigned grid, hipStream_t s);
 
-// Writes every edge held in the count pass's slots, one workgroup per tile (the write
-// stage of the two-stage build; tiles whose region needs two LDS chunks are expanded by
-// search_kernel<1>, larger ones written by it directly).
 // The positions in cell-list order (entry g: atom sid[g]), for the edge vectors: the
 // expansion then reads a tile's sources from a few contiguous runs instead of from all
 // over the caller's order.
@@ -1953,23 +2137,25 @@ __global__ void cell_pos_kernel(int64_t n, const int* __restrict__ sid, const vo
     }
 }
 
-// VT: void without vector / distance outputs, else their type.
-template <typename VT>
-__global__ __launch_bounds__(kBlock) void expand_kernel(SearchArgs a)
+// The ids to write for the cell-list entries.
+__global__ void cell_ids_kernel(int64_t n, const int* __restrict__ sid, const int64_t* __restrict__ out_ids,
+                                int* __restrict__ wid)
 {
-    // Tiles in reverse output order: the count stage wrote the slots in output order, so the
-    // last tiles' slots are the likeliest still in the memory-side cache when this kernel
-    // starts (C5 write stage 2.78 -> 2.70 ms, a uniform 1.25M-atom box 0.87 -> 0.82 ms).
-    // Each tile still writes its own output range.
-    const int64_t ord = (int64_t)gridDim.x - 1 - blockIdx.x;
-    if (a.tfix[ord] & (kFixChunked | kFix2)) return;
-    if constexpr (std::is_void<VT>::value) {
-        __shared__ ExpandLds sh;
-        expand_one<kCap>(a, sh, ord);
-    } else {
-        __shared__ ExpandVLds<VT> sh;
-        expand_one<kCap, VT>(a, sh, ord, &sh.vs);
-    }
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (g < n) wid[g] = (int)out_ids[sid[g]];
+}
+
+// The write stage: every edge the count pass left as row words, S workgroups per tile.
+// VT: the type of vector / distance outputs written in groups, else void.
+template <typename VT, bool GROUPS>
+__global__ __launch_bounds__(kBlock, expand_waves<VT>) void expand_kernel(SearchArgs a, int S)
+{
+    __shared__ ExpandLds<VT, GROUPS> sh;
+    int64_t ord;
+    int s;
+    part_of(blockIdx.x, a.ntiles, S, &ord, &s);
+    const int skew = GROUPS ? (int)(kSkewMax - (((uintptr_t)a.out_dst >> 3) & (kSkewMax - 1))) & (kSkewMax - 1) : 0;
+    expand_part<VT, GROUPS>(a, sh, ord, s, S, skew);
 }
 
 // ---------------------------------------------------------------- all-pairs fallback
@@ -2129,8 +2315,8 @@ struct StageTimer {
         (void)hipEventSynchronize(ev[n - 1]);
         float total = 0;
         fprintf(stderr, "[radius_graph_pbc profile] %s: N=%lld targets=%lld bins=%dx%dx%d tiles=%lld "
-                        "(%dx%dx%d bins) K=%d%s", call, (long long)p.n, (long long)p.nt, p.nb[0], p.nb[1],
-                p.nb[2], (long long)p.ntiles, p.T[0], p.T[1], p.T[2], p.K, p.brute ? " all-pairs" : "");
+                        "(%dx%dx%d bins) Kw=%d%s", call, (long long)p.n, (long long)p.nt, p.nb[0], p.nb[1],
+                p.nb[2], (long long)p.ntiles, p.T[0], p.T[1], p.T[2], p.Kw, p.brute ? " all-pairs" : "");
         if (capacity >= 0) fprintf(stderr, " edge capacity=%lld", (long long)capacity);
         fprintf(stderr, "\n");
         for (int i = 1; i < n; ++i) {
@@ -2244,6 +2430,14 @@ SearchArgs search_args(const Plan& p, const void* pos, void* ws)
     }
     a.tb = p.tb;
     a.nregion = p.nregion;
+    a.inv_R0 = 1.0f / (float)p.R[0];
+    a.inv_R01 = 1.0f / (float)(p.R[0] * p.R[1]);
+    a.wrap1 = 1;
+    for (int d = 0; d < 3; ++d) {
+        a.inv_T[d] = 1.0f / (float)p.T[d];
+        // (a region bin runs from -P to ntl T - 1 + P, and ntl T < nb + T)
+        if (p.pbc[d] && p.nb[d] < p.T[d] + p.P[d]) a.wrap1 = 0;
+    }
     a.xsplit = p.ntiles <= kSortTilesMax;  // (the per-bin sort above keeps bins in id order)
     a.ntiles = p.ntiles;
     a.toff = p.toff; a.hi_off = p.hi_off; a.lo_bits = p.lo_bits;
@@ -2264,13 +2458,19 @@ SearchArgs search_args(const Plan& p, const void* pos, void* ws)
     a.tfix = at<int>(ws, p.o_tfix);
     a.tbase = at<int64_t>(ws, p.o_tbase);
     a.totals = at<int64_t>(ws, p.o_tot);
-    // slot rows: one per target, or per atom when the targets are the atoms with ids < nt
+    // word rows: one per target, or per atom when the targets are the atoms with ids < nt
     // (every atom of a tile is then a lane)
-    const int64_t nrow = p.nrow;
-    a.slot = at<uint16_t>(ws, p.o_slot);
-    a.K = p.K;
-    a.nslot = nrow;
-    a.align_max_edges = -1;  // (set by the write call, which knows the outputs)
+    a.mid = p.mid; a.band = p.band; a.low = p.low;
+    a.words = at<uint32_t>(ws, p.o_slot);
+    a.nw = at<uint8_t>(ws, p.o_nw);
+    a.Kw = p.Kw;
+    a.nrow = p.nrow;
+    a.map = at<int2>(ws, p.o_map);
+    a.mapcap = p.mapcap;
+    // (64 tiles or more share a pool: their sizes even out; 128 bytes each fit 8 per tile)
+    a.npools = (int)std::max<int64_t>(1, std::min<int64_t>(64, p.ntiles / 64));
+    a.tmap = at<int2>(ws, p.o_wgb);  // (free once the atoms and targets are sorted)
+    a.wid = a.sid;
     a.ntarg = p.nt;
     // the prefix test runs with the tile-level sort only (the per-bin fallback sorts the
     // explicit targets as listed)
@@ -2332,7 +2532,7 @@ void launch_sort(const Plan& p, const void* pos, const int64_t* target_idx, void
         int* wgb = at<int>(ws, p.o_wgb);
         hipLaunchKernelGGL(tile_rank_kernel, dim3((unsigned)std::min<int64_t>(nblocks(p.ntiles), 2048)),
                            dim3(256), 0, s, g, p.ntiles, at<int>(ws, p.o_tor), at<int>(ws, p.o_rot), tcnt,
-                           p.ntiles, totals);
+                           p.ntiles, totals, at<int64_t>(ws, p.o_tbase));
         // 2. wrap, bin key and cell-list record of every atom
         hipLaunchKernelGGL(bin_atoms_kernel, dim3(nblocks(p.n)), dim3(256), 0, s, g, pos, p.f64, p.n,
                            (const int*)at<int>(ws, p.o_rot), at<uint32_t>(ws, p.o_key),
@@ -2417,7 +2617,8 @@ void launch_sort(const Plan& p, const void* pos, const int64_t* target_idx, void
     } else {
     // 1. Morton rank of the tiles (and cleared bin counts)
     hipLaunchKernelGGL(tile_rank_kernel, dim3((unsigned)std::min<int64_t>(nblocks(p.nbins), 2048)), dim3(256),
-                       0, s, g, p.ntiles, at<int>(ws, p.o_tor), at<int>(ws, p.o_rot), bcnt, p.nbins, totals);
+                       0, s, g, p.ntiles, at<int>(ws, p.o_tor), at<int>(ws, p.o_rot), bcnt, p.nbins, totals,
+                       at<int64_t>(ws, p.o_tbase));
     // 2-5. counting sort of the atoms into SFC-ordered bins (per-bin device atomics)
     hipLaunchKernelGGL(bin_atoms_kernel, dim3(nblocks(p.n)), dim3(256), 0, s, g, pos, p.f64, p.n,
                        (const int*)at<int>(ws, p.o_rot), at<uint32_t>(ws, p.o_key),
@@ -2485,7 +2686,7 @@ size_t dg_graph_workspace_size(const dg_graph_desc* desc)
     return p.ws_bytes;
 }
 
-// The count stage; without slots (counts only) the sweep records no neighbour lists, and a
+// The count stage; without slots (counts only) the sweep records no row words, and a
 // dg_graph_write that follows writes every tile from its fix-up pass instead.
 static dg_status count_stage(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
                              void* ws, size_t ws_bytes, int32_t* counts_out, bool slots, hipStream_t s)
@@ -2520,7 +2721,7 @@ static dg_status count_stage(const dg_graph_desc* desc, const void* pos, const i
     // 6. degrees
     SearchArgs a = search_args(p, pos, ws);
     a.counts_user = counts_out;
-    if (!slots) a.slot = nullptr;
+    if (!slots) a.words = nullptr;
     launch_count_kernel(a, (unsigned)p.ntiles, s);
     clk.mark("count");
     // 7. tile offsets in output order, and the total
@@ -2606,12 +2807,12 @@ dg_status dg_graph_write_ids(const dg_graph_desc* desc, const void* pos, const i
     a.out_vec = edge_vec; a.out_dist = edge_dist; a.vout_f64 = vec_dtype == DG_F64;
     a.capacity = capacity;
     a.out_ids = out_ids;
-    {
-        const double slot_bytes = 2.0 * (double)p.K * (double)a.nslot;
-        const double bpe = 28.0 + (edge_vec ? (vec_dtype == DG_F64 ? 24.0 : 12.0) : 0.0) +
-                           (edge_dist ? (vec_dtype == DG_F64 ? 8.0 : 4.0) : 0.0);
-        const double room = kAlignBudget - slot_bytes;
-        a.align_max_edges = room > 0 ? (int64_t)(room / (kAlignOutShare * bpe)) : -1;
+    if (out_ids) {
+        // the ids to write in cell-list order (over the sort's scratch), so that the expansion
+        // reads them from a tile's few runs
+        int* wid = at<int>(ws, p.o_arr);
+        hipLaunchKernelGGL(cell_ids_kernel, dim3(nblocks(p.n)), dim3(256), 0, s, (int64_t)p.n, a.sid, out_ids, wid);
+        a.wid = wid;
     }
     StageTimer clk(s);
     clk.mark("start");
@@ -2624,12 +2825,20 @@ dg_status dg_graph_write_ids(const dg_graph_desc* desc, const void* pos, const i
         hipLaunchKernelGGL(cell_pos_kernel, dim3(nblocks(p.n, 256)), dim3(256), 0, s, (int64_t)p.n,
                            (const int*)a.sid, pos, p.f64, (void*)a.cpos);
     }
+    // parts per tile, from the edges expected: as many blocks to a part (whose setup costs about
+    // as much as a block) as leave the chip a few rounds of workgroups
+    const double per_tile = p.deg * (double)p.nt / (double)p.ntiles;
+    const double part = kSub * std::min(std::max(floor((double)p.ntiles * per_tile / ((double)kSub * kPartsWanted)), 1.0), kPartBlocks);
+    const int parts = (int)std::min(std::max(ceil(per_tile / part), 1.0), 64.0);
+    const dim3 grid((unsigned)(p.ntiles * parts));
     if (vec16 && a.vout_f64)
-        hipLaunchKernelGGL(expand_kernel<double>, dim3((unsigned)p.ntiles), dim3(kBlock), 0, s, a);
+        hipLaunchKernelGGL((expand_kernel<double, true>), grid, dim3(kBlock), 0, s, a, parts);
     else if (vec16)
-        hipLaunchKernelGGL(expand_kernel<float>, dim3((unsigned)p.ntiles), dim3(kBlock), 0, s, a);
+        hipLaunchKernelGGL((expand_kernel<float, true>), grid, dim3(kBlock), 0, s, a, parts);
+    else if (vec)
+        hipLaunchKernelGGL((expand_kernel<void, false>), grid, dim3(kBlock), 0, s, a, parts);
     else
-        hipLaunchKernelGGL(expand_kernel<void>, dim3((unsigned)p.ntiles), dim3(kBlock), 0, s, a);
+        hipLaunchKernelGGL((expand_kernel<void, true>), grid, dim3(kBlock), 0, s, a, parts);
     clk.mark("write (slot expansion)");
     hipLaunchKernelGGL(search_kernel<1>, dim3((unsigned)std::min<int64_t>(p.ntiles, kFixGrid)), dim3(kBlock), 0, s, a);
     clk.mark("write (fix-up)");
@@ -2653,7 +2862,7 @@ dg_status dg_graph_build(const dg_graph_desc* desc, const void* pos, const int64
                          void* edge_dist, int32_t vec_dtype, hipStream_t s)
 {
     // the write pass reads only device-side results of the count pass (per-tile offsets,
-    // slots), so the two run back to back with no host round trip
+    // row words), so the two run back to back with no host round trip
     dg_status st = dg_graph_count(desc, pos, target_idx, ws, ws_bytes, counts_out, s);
     if (st != DG_OK) return st;
     return dg_graph_write(desc, pos, target_idx, ws, ws_bytes, capacity, edge_src, edge_dst,
@@ -2664,7 +2873,7 @@ dg_status dg_graph_build(const dg_graph_desc* desc, const void* pos, const int64
 
 // ---------------------------------------------------------------- allocation-free build
 // A device-resident workspace for dg_graph_build_noalloc: the build's whole workspace
-// (cell list, slots, tile tables, totals) lives in this array, one copy per GPU, held from
+// (cell list, row words, tile tables, totals) lives in this array, one copy per GPU, held from
 // the library's load until the process ends.  Host code never names the array itself (its
 // host-side symbol is no device address): it uses the address hipGetSymbolAddress
 // returns on each device, kept in g_scratch_ptr.

@@ -47,6 +47,7 @@ struct Plan {
     float hi = 0, lo_in = 0, tiny = 0;
     float toff = 0, hi_off = 0;  // the same bounds on d2 - toff (see plan_grid)
     uint32_t lo_bits = 0;        // bits of the fp32 bound lo_off on d2 - toff
+    float mid = 0, band = 0, low = 0;  // the count pass's bounds on d2 - mid (see plan_grid)
     // workspace layout (byte offsets)
     size_t o_key, o_rank, o_rec, o_bcnt, o_bstart, o_sid, o_spos, o_sflr, o_inv;
     size_t o_cpos;  // write stage, vector outputs: positions in cell-list order (over key .. rec)
@@ -55,9 +56,12 @@ struct Plan {
     size_t o_tarr;                   // the same sort of explicit targets: their tile buckets
     size_t o_stmp;                   // segment-sort scratch (8 B per atom or target)
     size_t o_tkey, o_trank, o_tbcnt, o_tbstart, o_tslot, o_tsidx, o_tcaller;
-    size_t o_cnt, o_ttot, o_tfix, o_tbase, o_part, o_tot, o_slot;
-    int K = 0;              // neighbour slot entries per target
-    int64_t nrow = 0;       // slot rows (group-major row length)
+    size_t o_cnt, o_ttot, o_tfix, o_tbase, o_part, o_tot, o_slot, o_nw, o_map;
+    int K = 0;              // sizes the write stage's lists: 2 K bytes per target in all
+    int Kw = 0;             // row words per target, of those bytes
+    double deg = 0;         // expected degree at the mean density
+    int64_t mapcap = 0;     // region map entries: the bytes left
+    int64_t nrow = 0;       // targets padded (group-major row length)
     size_t ws_bytes = 0;
 };
 
@@ -230,15 +234,22 @@ inline void plan_grid(Plan& p)
     if ((double)p.hi_off < hi2) p.hi_off = nextafterf(p.hi_off, INFINITY);
     p.hi_off = nextafterf(p.hi_off, INFINITY);
 
-    // Neighbour slot per target: the expected degree at the mean density with ample
-    // headroom (targets past it are swept a second time in the write pass).
+    // The count pass evaluates d2'' = fl(dz^2 + (dy^2 + (dx^2 - mid))), mid = fl(r^2): the sign
+    // bit is the edge test.  As for d2' above, each of its roundings is at most u mid wherever
+    // d2 is below 2 r^2 (past that the sign is certain), so it lies within the band of the exact
+    // d2 - mid; |mid - r^2| <= u mid.  Near zero the offset costs the small distances their
+    // precision: up to low, 8 u mid above tiny, the exact test decides (and drops the self pair).
+    p.mid = (float)p.r2;
+    p.band = nextafterf((float)((band + 8.0 * u * p.r2) * (1.0 + 1e-6)), INFINITY);
+    p.low = nextafterf((float)((double)p.tiny * (1.0 + 1e-6) + 16.0 * u * p.r2 - (double)p.mid), INFINITY);
+
+    // Bytes per target that the write stage's lists may take (row words and region map share
+    // them): from the expected degree at the mean density, with ample headroom.
     const double vol = fabs(p.C[0] * (p.C[4] * p.C[8] - p.C[5] * p.C[7]) -
                             p.C[1] * (p.C[3] * p.C[8] - p.C[5] * p.C[6]) +
                             p.C[2] * (p.C[3] * p.C[7] - p.C[4] * p.C[6]));
-    const double deg = (double)p.n / vol * (4.0 / 3.0) * 3.14159265358979 * p.r * p.r * p.r;
-    // (1.5x + 48: the headroom also covers a density up to about twice the mean in part
-    // of the cell, as in a two-phase slab; unused groups of a slot are never touched)
-    double k = 1.5 * deg + 48.0;
+    p.deg = (double)p.n / vol * (4.0 / 3.0) * 3.14159265358979 * p.r * p.r * p.r;
+    double k = 1.5 * p.deg + 48.0;
     k = std::min(std::max(k, 32.0), 2048.0);
     p.K = ((int)k + 7) & ~7;
 }
@@ -278,17 +289,35 @@ inline void plan_layout(Plan& p)
     p.o_tarr = take(p.subset ? 8 * nt : 0);
     p.o_tsidx = take(p.subset ? 4 * nt : 0);
     p.o_tcaller = take(p.subset ? 4 * nt : 0);
-    // scratch of the segment sort (tile buckets, bins of the per-bin sort): one entry per
-    // atom or target
-    p.o_stmp = take(8 * std::max(n, nt));
-    // per-target counts and slots: one row per target, or per atom when explicit targets
+    // per-target counts and row words: one row per target, or per atom when explicit targets
     // turn out to be the atoms 0 .. nt - 1 (the count then runs over every atom of a tile)
     // (rows padded to 256 targets: the group rows of a row length of 2 mod 4 targets, e.g.
     // C5's 4,436,018 atoms, made the expansion 5 % slower, 3.02 against 2.87 ms)
     const size_t nrow = (std::max(n, nt) + 255) / 256 * 256;
     p.nrow = (int64_t)nrow;
     p.o_cnt = take(4 * nrow);
+    // 2 K bytes per target: the row words, their counts, and the region map in what is left;
+    // the map goes on over the scratch of the segment sort (tile buckets, bins of the per-bin
+    // sort: one entry per atom or target), which is free once the atoms are sorted
     p.o_slot = take(2 * (size_t)p.K * nrow);
+    p.o_stmp = take(8 * std::max(n, nt));
+    {
+        // The region map first: an atom is in the regions of ntl R / nb tiles per axis (on
+        // average over the bins; the tenth covers a density that favours the bins in more
+        // regions).  Then the row words: the stencil rows expected to hold an edge, with headroom
+        // for a density above the mean (a two-phase cell), and the second words of long rows (a
+        // swept row holds about twice the candidates it has edges).  A tile past the map, or a
+        // target past its words, is written by the fix-up pass.
+        double regions = 1.1 * (double)n;
+        for (int d = 0; d < 3; d++) regions *= (double)p.ntl[d] * p.R[d] / p.nb[d];
+        const double rows = std::min(4096.0, (2.0 * p.P[1] + 1.0) * (2.0 * p.P[2] + 1.0));
+        const double want = 4.0 + 1.35 * rows * (1.0 - exp(-p.deg / (0.86 * rows))) + 0.25 * p.deg;
+        const double room = ((double)(o - p.o_slot) - 8.0 * regions - (double)nrow - 1024.0) / (4.0 * (double)nrow);
+        p.Kw = std::max(8, (int)std::min({want, room, 248.0}) & ~3);
+    }
+    p.o_nw = align_up(p.o_slot + 4 * (size_t)p.Kw * nrow);
+    p.o_map = align_up(p.o_nw + nrow);
+    p.mapcap = o > p.o_map ? std::min<int64_t>((int64_t)((o - p.o_map) / 8), 0x7fffff00LL) : 0;
     p.o_ttot = take(4 * std::max(ntl, nt));
     p.o_tfix = take(4 * ntl);
     p.o_tbase = take(8 * (std::max(ntl, nt) + 1));

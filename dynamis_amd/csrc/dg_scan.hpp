@@ -24,6 +24,61 @@ __device__ __forceinline__ T wave_incl_scan(T x)
     return x;
 }
 
+// The same for an int, by data-parallel moves between lanes (no LDS round trips): within rows
+// of 16 lanes by shifts, then each row's sum to the rows after it.  All 64 lanes are active.
+__device__ __forceinline__ int wave_incl_scan_dpp(int x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1, 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
+    return x;
+}
+
+// Exclusive scan of an int across a workgroup of NT threads, with one barrier: the caller has a
+// barrier between two uses of s_w (NT / 64 ints).
+template <int NT>
+__device__ __forceinline__ int block_excl_scan_dpp(int v, int* s_w, int* total)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int x = wave_incl_scan_dpp(v);
+    if (lane == 63) s_w[w] = x;
+    __syncthreads();
+    int before = 0, tot = 0;
+#pragma unroll
+    for (int i = 0; i < NT / 64; ++i) {
+        const int s = s_w[i];
+        before += i < w ? s : 0;
+        tot += s;
+    }
+    *total = tot;
+    return before + x - v;
+}
+
+// Two of them at once.
+template <int NT>
+__device__ __forceinline__ int2 block_excl_scan2(int2 v, int2* s_w, int* total_x, int* total_y)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int x = wave_incl_scan_dpp(v.x), y = wave_incl_scan_dpp(v.y);
+    if (lane == 63) s_w[w] = make_int2(x, y);
+    __syncthreads();
+    int2 before = make_int2(0, 0), tot = make_int2(0, 0);
+#pragma unroll
+    for (int i = 0; i < NT / 64; ++i) {
+        const int2 s = s_w[i];
+        before.x += i < w ? s.x : 0;
+        before.y += i < w ? s.y : 0;
+        tot.x += s.x;
+        tot.y += s.y;
+    }
+    *total_x = tot.x;
+    *total_y = tot.y;
+    return make_int2(before.x + x - v.x, before.y + y - v.y);
+}
+
 // Exclusive scan across a workgroup of NT threads (NT multiple of 64).  s_w holds
 // NT/64 values.  Returns the exclusive prefix; *total receives the workgroup sum.
 template <typename T, int NT>

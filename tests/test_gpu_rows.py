@@ -1,0 +1,96 @@
+"""The count pass's row words and the expansion's blocks at their edges: stencil rows of as many
+candidates as one word, one sweep piece or one mask hold, and one more; pairs at distances around
+the exclusion of coincident atoms; target ids that start anywhere in a 128-byte line, and tiles
+that start and end anywhere in a block.  Results are whole numbers, compared with the CPU oracle
+(or, byte for byte, with the aligned build)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from dynamis_amd import _lib as L
+from dynamis_amd import configs
+from dynamis_amd.dynamis_state import dynamis_state_impl as impl
+
+pytestmark = pytest.mark.gpu
+
+
+def _parity(pos, cell, pbc, r, dev):
+    ei, co, _, cnt = impl.radius_graph_pbc_ex(torch.from_numpy(pos).to(dev), torch.from_numpy(cell),
+                                              torch.tensor(pbc), r, 0, False)
+    torch.cuda.synchronize()
+    used = cell.astype(pos.dtype).astype(np.float64)
+    o = oracle.radius_graph(pos, used, pbc, float(np.float32(r)))
+    assert np.array_equal(cnt.cpu().numpy(), o["counts"])
+    got = oracle.canonical_sort(ei[0].cpu().numpy(), ei[1].cpu().numpy(), co.cpu().numpy().astype(np.int64))
+    for a, b in zip(got, oracle.canonical_sort(o["src"], o["dst"], o["shift"])):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("cell", ["cubic", "sheared", "general"])
+@pytest.mark.parametrize("k", [1, 2, 4, 5, 19, 20, 21, 27, 28, 29, 40, 41, 56, 57, 130])
+def test_rows_of_k_candidates(cuda, cell, k):
+    """k atoms side by side along x (one stencil row holds them all) among a few others."""
+    print(f"\n[case] rows k={k} {cell}", flush=True)
+    rng = np.random.default_rng(k)
+    pos = rng.uniform(0.0, 30.0, (60, 3))
+    line = np.full((k, 3), 15.0) + rng.uniform(-0.05, 0.05, (k, 3))
+    line[:, 0] += rng.permutation(np.linspace(-1.0, 1.0, k))
+    C = np.eye(3) * 30.0
+    if cell == "sheared":
+        C[1, 0], C[2, 0], C[2, 1] = 6.0, -4.0, 5.0
+    elif cell == "general":
+        C[0, 1], C[1, 2], C[2, 0] = 5.0, -4.0, 3.0
+    pos = np.concatenate([pos, line])[rng.permutation(60 + k)].astype(np.float32)
+    _parity(pos, C, (True, True, True), 5.0, cuda)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_close_pairs(cuda, dtype):
+    """Pairs at distances around 1e-4 (the exclusion of coincident atoms), duplicates included,
+    inside a bin and across bins and cell faces."""
+    print(f"\n[case] close pairs {np.dtype(dtype)}", flush=True)
+    rng = np.random.default_rng(3)
+    base = rng.uniform(0.0, 24.0, (200, 3))
+    base[:8, 0] = 0.0
+    base[8:16] = np.round(base[8:16] / 2.4) * 2.4
+    seps = np.array([0.0, 1e-6, 5e-5, 9.9e-5, 1e-4, 1.01e-4, 2e-4, 1e-3, 3e-3, 1e-2])
+    d = rng.normal(size=(200, 3))
+    d *= (seps[np.arange(200) % len(seps)] / np.linalg.norm(d, axis=1))[:, None]
+    pos = np.concatenate([base, base + d]).astype(dtype)
+    _parity(pos, np.eye(3) * 24.0, (True, True, True), 5.0, cuda)
+
+
+def _build(pos, cell, dev, r, cap, skew):
+    """dg_graph_build with the target ids `skew` entries into an array that starts on a line, and
+    guard values around every output."""
+    lib = L.lib()
+    d = impl._desc(pos, cell, torch.tensor([True, True, True]), impl._r32(r), None)
+    wsb = lib.dg_graph_workspace_size(d)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+    cnt = torch.empty(pos.size(0), dtype=torch.int32, device=dev)
+    src = torch.full((cap + 64,), -7, dtype=torch.int64, device=dev)
+    dst = torch.full((cap + 64,), -7, dtype=torch.int64, device=dev)
+    sh = torch.full((cap + 64, 3), -7.0, dtype=torch.float32, device=dev)
+    st = lib.dg_graph_build(d, L.ptr(pos), None, L.ptr(ws), wsb, cap, L.ptr(cnt), L.ptr(src),
+                            L.ctypes.c_void_p(dst.data_ptr() + 8 * skew), L.ptr(sh), None, None, L.DG_F32,
+                            L.stream_of(dev))
+    L.check(st, "dg_graph_build")
+    E, fl = L._i64(0), L._i64(0)
+    L.check(lib.dg_graph_read_totals(d, L.ptr(ws), E, fl, L.stream_of(dev)), "totals")
+    return int(E.value), src, dst, sh
+
+
+@pytest.mark.parametrize("n", [40, 700, 3001, 20011])
+def test_target_ids_anywhere_in_a_line(cuda, n):
+    print(f"\n[case] skewed target ids n={n}", flush=True)
+    b = configs.uniform(n, density=0.08, seed=n, dtype=np.float32, radius=5.0)
+    pos, cell = torch.from_numpy(b.pos).to(cuda), torch.from_numpy(b.cell)
+    E, src0, dst0, sh0 = _build(pos, cell, cuda, b.radius, 200 * n, 0)
+    assert E > 0 and bool((src0[E:] == -7).all()) and bool((dst0[E:] == -7).all()) and bool((sh0[E:] == -7).all())
+    for skew in range(1, 17):
+        e, src, dst, sh = _build(pos, cell, cuda, b.radius, 200 * n, skew)
+        assert e == E
+        assert torch.equal(src, src0) and torch.equal(sh, sh0)
+        assert torch.equal(dst[skew:skew + E], dst0[:E])
+        assert bool((dst[:skew] == -7).all()) and bool((dst[skew + E:] == -7).all())
