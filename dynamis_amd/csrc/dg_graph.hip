@@ -2829,7 +2829,7 @@ dg_status dg_graph_write_ids(const dg_graph_desc* desc, const void* pos, const i
     // as much as a block) as leave the chip a few rounds of workgroups
     const double per_tile = p.deg * (double)p.nt / (double)p.ntiles;
     const double part = kSub * std::min(std::max(floor((double)p.ntiles * per_tile / ((double)kSub * kPartsWanted)), 1.0), kPartBlocks);
-    const int parts = (int)std::min(std::max(ceil(per_tile / part), 1.0), 64.0);
+    const int parts = (int)std::min({std::max(ceil(per_tile / part), 1.0), 64.0, floor(2147483647.0 / (double)p.ntiles)});
     const dim3 grid((unsigned)(p.ntiles * parts));
     if (vec16 && a.vout_f64)
         hipLaunchKernelGGL((expand_kernel<double, true>), grid, dim3(kBlock), 0, s, a, parts);

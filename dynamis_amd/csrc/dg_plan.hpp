@@ -312,8 +312,9 @@ inline void plan_layout(Plan& p)
         for (int d = 0; d < 3; d++) regions *= (double)p.ntl[d] * p.R[d] / p.nb[d];
         const double rows = std::min(4096.0, (2.0 * p.P[1] + 1.0) * (2.0 * p.P[2] + 1.0));
         const double want = 4.0 + 1.35 * rows * (1.0 - exp(-p.deg / (0.86 * rows))) + 0.25 * p.deg;
-        const double room = ((double)(o - p.o_slot) - 8.0 * regions - (double)nrow - 1024.0) / (4.0 * (double)nrow);
-        p.Kw = std::max(8, (int)std::min({want, room, 248.0}) & ~3);
+        const double room = ((double)(o - p.o_slot) - 8.0 * regions - (double)nrow - 1024.0) /
+                            (4.0 * (double)std::max<size_t>(nrow, 1));
+        p.Kw = (int)std::max(8.0, std::min({want, room, 248.0})) & ~3;
     }
     p.o_nw = align_up(p.o_slot + 4 * (size_t)p.Kw * nrow);
     p.o_map = align_up(p.o_nw + nrow);
