@@ -74,7 +74,7 @@ def _desc(pos, cell, pbc, radius, target_indices):
     d.pos_dtype = L.DG_F64 if pos.dtype == torch.float64 else L.DG_F32
     # The reference casts the cell to float32 (radius_graph.cpp:24); with float64
     # positions the cell is kept in float64.
-    c = cell.detach().to(device="cpu", dtype=pos.dtype).to(torch.float64).reshape(-1).tolist()
+    c = cell.detach().cpu().to(pos.dtype).to(torch.float64).reshape(-1).tolist()
     for k in range(9):
         d.cell[k] = c[k]
     pb = pbc.detach().to("cpu").to(torch.bool).tolist()
@@ -174,8 +174,9 @@ def build_batch(pos, cells, natoms, pbc, radius, max_num_neighbors=0):
     d.n_images = B
     d.n_atoms = pos.size(0)
     d.pos_dtype = L.DG_F64 if pos.dtype == torch.float64 else L.DG_F32
+    pb = pbc.detach().cpu().to(torch.bool).tolist()
     for k in range(3):
-        d.pbc[k] = 1 if bool(pbc[k]) else 0
+        d.pbc[k] = 1 if pb[k] else 0
     d.radius = _r32(radius)
     # the cell rounded to the position dtype, as the single-structure binding does
     # (radius_graph.cpp:24)

@@ -4,6 +4,7 @@ of every structure of the batch, with batch atom indices -- a batch of small str
 one launch sequence (``dynamis_state_impl.build_batch``), others one structure at a time."""
 from __future__ import annotations
 
+import numpy as np
 import torch
 
 from . import dynamis_state_impl as _impl
@@ -34,21 +35,19 @@ _BATCH_MS_PER_PAIR = 1.6e-8
 _BATCH_IMAGES_MEASURED = 6.0
 
 
-def _images_per_pair(cell, pbc, radius) -> float:
-    """prod over periodic axes of (2 r / d_face + 1) for one cell (rows = lattice vectors)."""
-    import numpy as np
-
-    c = np.asarray(cell, dtype=np.float64).reshape(3, 3)
-    vol = abs(float(np.dot(c[0], np.cross(c[1], c[2]))))
-    img = 1.0
-    for d in range(3):
-        if not pbc[d]:
-            continue
-        area = float(np.linalg.norm(np.cross(c[(d + 1) % 3], c[(d + 2) % 3])))
-        if vol <= 0.0 or area <= 0.0:
-            return float("inf")
-        img *= 2.0 * float(radius) / (vol / area) + 1.0
-    return img
+def _images_per_pair(cells, pbc, radius):
+    """prod over periodic axes of (2 r / d_face + 1), for one cell (rows = lattice vectors) or,
+    elementwise, for an array of cells: one array expression for a whole batch (cell by cell it
+    took 5 ms for 128 structures, ten times the batch's build)."""
+    c = np.asarray(cells, dtype=np.float64).reshape(-1, 3, 3)
+    normals = np.cross(c[:, [1, 2, 0]], c[:, [2, 0, 1]])  # a_j x a_k per axis
+    vol = np.abs(np.einsum("bi,bi->b", c[:, 0], normals[:, 0]))[:, None]
+    area = np.sqrt(np.einsum("bdi,bdi->bd", normals, normals))
+    ok = (vol > 0.0) & (area > 0.0)
+    with np.errstate(divide="ignore", invalid="ignore", over="ignore"):
+        img = np.where(ok, 2.0 * float(radius) * area / vol + 1.0, np.inf)
+    out = np.where(np.asarray(pbc, dtype=bool), img, 1.0).prod(axis=1)
+    return out if np.ndim(cells) == 3 else float(out[0])
 
 
 def _batch_in_one_pass(natoms, cells=None, pbc=(True, True, True), radius=6.0) -> bool:
@@ -57,12 +56,13 @@ def _batch_in_one_pass(natoms, cells=None, pbc=(True, True, True), radius=6.0) -
     if len(natoms) < 2 or max(natoms) > BATCH_MAX_ATOMS:
         return False
     if cells is None:
-        weights = [1.0] * len(natoms)
+        weights = 1.0
     else:
-        weights = [_images_per_pair(c, pbc, radius) / _BATCH_IMAGES_MEASURED for c in cells]
-        if max(weights) * _BATCH_IMAGES_MEASURED > BATCH_MAX_IMAGES:
+        images = _images_per_pair(np.asarray(cells, dtype=np.float64).reshape(-1, 3, 3), pbc, radius)
+        if images.max() > BATCH_MAX_IMAGES:
             return False
-    pairs = sum(n * n * w for n, w in zip(natoms, weights))
+        weights = images / _BATCH_IMAGES_MEASURED
+    pairs = float((np.asarray(natoms, dtype=np.float64) ** 2 * weights).sum())
     return _BATCH_MS + _BATCH_MS_PER_PAIR * pairs < _LOOP_MS_PER_STRUCTURE * len(natoms)
 
 
@@ -76,7 +76,8 @@ def radius_graph_pbc_cuda(data, radius: float, max_num_neighbors_threshold: int,
     Mixed PBC across the batch raises RuntimeError (reference :37-48).
     """
     if pbc is None:
-        data_pbc = torch.atleast_2d(data.pbc)
+        # (on the host: one copy instead of five small kernels and the waits for their results)
+        data_pbc = torch.atleast_2d(data.pbc.detach().cpu())
         all_true = torch.all(data_pbc, dim=0)
         all_false = torch.all(~data_pbc, dim=0)
         mixed = ~(all_true | all_false)
