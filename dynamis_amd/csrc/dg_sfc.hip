@@ -155,7 +155,10 @@ __global__ void keys_kernel(const float* __restrict__ pos, int64_t n, int curve,
 //                        permutation;
 //   per byte q = 0..7:
 //     rs_hist_kernel<q>  each tile's digit counts, digit-major (hist[d * ntiles + t]);
-//     device scan of hist (digit-major: each tile's output base per digit)
+//     rs_rows_kernel<q>  one workgroup per digit scans the digit's counts over the tiles, and
+//                        leaves the digit's total (the pass adds up the totals itself: one
+//                        short launch where a scan of the whole array took two, 258 -> 222 us
+//                        for the weighted partition of 1M atoms)
 //     rs_pass_kernel<q>  each tile ranks its keys stably by digit (eight ballots per 64
 //                        keys and per-wave running counts) and writes each digit's run
 //                        contiguously through LDS: keys and int32 positions, or, in the last
@@ -285,6 +288,38 @@ __global__ __launch_bounds__(kRsBlock) void rs_hist_kernel(const int64_t* __rest
     hist[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = h[threadIdx.x];
 }
 
+// Row d of hist (the counts of digit d, tile by tile) scanned into offs, its sum into total[d].
+template <int Q>
+__global__ __launch_bounds__(kRsBlock) void rs_rows_kernel(const RsCtl* __restrict__ ctl, int64_t ntiles,
+                                                           const int* __restrict__ hist, int* __restrict__ offs,
+                                                           int* __restrict__ total)
+{
+    if (!ctl->pass[Q].run) return;
+    __shared__ int s_w[kRsBlock / 64];
+    constexpr int kPer = 4;
+    const int64_t row = (int64_t)blockIdx.x * ntiles;
+    int carry = 0;
+    for (int64_t t0 = 0; t0 < ntiles; t0 += kPer * kRsBlock) {
+        const int64_t t = t0 + kPer * threadIdx.x;
+        int c[kPer], sum = 0;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            c[u] = t + u < ntiles ? hist[row + t + u] : 0;
+            sum += c[u];
+        }
+        int tot;
+        int ex = carry + block_excl_scan_dpp<kRsBlock>(sum, s_w, &tot);
+        __syncthreads();  // (before the next round writes s_w)
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            if (t + u < ntiles) offs[row + t + u] = ex;
+            ex += c[u];
+        }
+        carry += tot;
+    }
+    if (threadIdx.x == 0) total[blockIdx.x] = carry;
+}
+
 struct RsScatterLds {
     union {
         uint64_t k[kRsTile];  // the tile's keys in slot (digit) order
@@ -294,14 +329,16 @@ struct RsScatterLds {
     int glob[256];             // output index of slot 0 of each digit's run, for this tile
     int wc[kRsBlock / 64][256];  // per wave: running count per digit, then its first slot
     int w32[kRsBlock / 64];
+    int d32[kRsBlock / 64];
 };
 
-// Pass over byte Q.  offs: the exclusive scan of this pass's tile counts (digit-major).
+// Pass over byte Q.  offs: each digit's counts in the tiles before a tile (digit-major); total:
+// each digit's count.
 template <int Q>
 __global__ __launch_bounds__(kRsBlock) void rs_pass_kernel(
     const int64_t* __restrict__ ukeys, int64_t n, int64_t* __restrict__ kb1, int64_t* __restrict__ kb2,
     int32_t* __restrict__ vb1, int32_t* __restrict__ vb2, int64_t* __restrict__ perm,
-    const RsCtl* __restrict__ ctl, const int* __restrict__ offs)
+    const RsCtl* __restrict__ ctl, const int* __restrict__ offs, const int* __restrict__ total)
 {
     constexpr int shift = 8 * Q;
     const RsPass P = ctl->pass[Q];
@@ -336,7 +373,8 @@ __global__ __launch_bounds__(kRsBlock) void rs_pass_kernel(
     }
     // this tile's output base per digit (independent of the ranking below, so its load
     // overlaps it): the keys of lower digits plus this digit's keys in the tiles before
-    const int before_t = offs[(int64_t)threadIdx.x * ntiles + t];
+    int before_t = offs[(int64_t)threadIdx.x * ntiles + t];
+    const int mine = total[threadIdx.x];
 #pragma unroll
     for (int u = 0; u < kRsPer; ++u) {
         const int i = w * kRsWaveKeys + u * 64 + lane;
@@ -366,8 +404,9 @@ __global__ __launch_bounds__(kRsBlock) void rs_pass_kernel(
         const int d = threadIdx.x;
         int c = 0;
         for (int k = 0; k < kRsBlock / 64; ++k) c += S.wc[k][d];
-        int tot;
-        const int ex = block_excl_scan<int, kRsBlock>(c, S.w32, &tot);
+        int tot, all;
+        before_t += block_excl_scan_dpp<kRsBlock>(mine, S.d32, &all);
+        const int ex = block_excl_scan_dpp<kRsBlock>(c, S.w32, &tot);
         int at = ex;
         for (int k = 0; k < kRsBlock / 64; ++k) {
             const int ck = S.wc[k][d];
@@ -733,7 +772,7 @@ dg_status launch_ok(const char* what)
 }
 
 struct SortLayout {
-    size_t o_k0, o_v0, o_k1, o_v1, o_part, o_ctl, o_hist, o_offs, o_spart, total;
+    size_t o_k0, o_v0, o_k1, o_v1, o_part, o_ctl, o_hist, o_offs, o_rows, total;
     int nblocks, nparts;
 };
 
@@ -753,8 +792,8 @@ SortLayout sort_layout(int64_t n)
     L.o_part = take(16 * (size_t)L.nparts);
     L.o_ctl = take(sizeof(RsCtl));
     L.o_hist = take(4 * nh);
-    L.o_offs = take(4 * (nh + 1));
-    L.o_spart = take(4 * (nh / kScanTile + 2));
+    L.o_offs = take(4 * nh);
+    L.o_rows = take(4 * 256);
     L.total = o;
     return L;
 }
@@ -828,16 +867,17 @@ dg_status dg_sfc_order(const int64_t* keys, int64_t n, int64_t* perm, void* ws, 
     RsCtl* ctl = (RsCtl*)(w + L.o_ctl);
     int* hist = (int*)(w + L.o_hist);
     int* offs = (int*)(w + L.o_offs);
+    int* total = (int*)(w + L.o_rows);
     hipLaunchKernelGGL(rs_span_kernel, dim3((unsigned)L.nparts), dim3(256), 0, s, keys, n, part);
     hipLaunchKernelGGL(rs_plan_kernel, dim3(1), dim3(256), 0, s, (const unsigned long long*)part, L.nparts, ctl);
     const dim3 grid((unsigned)L.nblocks), blk(kRsBlock);
-    // (a skipped pass's scan runs over stale counts; nothing reads its result)
 #define DG_RS_PASS(q)                                                                                  \
     hipLaunchKernelGGL(rs_hist_kernel<q>, grid, blk, 0, s, keys, n, (const int64_t*)kb1, (const int64_t*)kb2, \
                        (const RsCtl*)ctl, hist);                                                         \
-    excl_scan<int, int>(hist, (int64_t)L.nblocks * 256, offs, (int*)(w + L.o_spart), s);               \
+    hipLaunchKernelGGL(rs_rows_kernel<q>, dim3(256), blk, 0, s, (const RsCtl*)ctl, (int64_t)L.nblocks,  \
+                       (const int*)hist, offs, total);                                                  \
     hipLaunchKernelGGL(rs_pass_kernel<q>, grid, blk, 0, s, keys, n, kb1, kb2, vb1, vb2, perm,           \
-                       (const RsCtl*)ctl, (const int*)offs)
+                       (const RsCtl*)ctl, (const int*)offs, (const int*)total)
     DG_RS_PASS(0);
     DG_RS_PASS(1);
     DG_RS_PASS(2);
