@@ -157,7 +157,7 @@ __global__ void keys_kernel(const float* __restrict__ pos, int64_t n, int curve,
 //     rs_hist_kernel<q>  each tile's digit counts, digit-major (hist[d * ntiles + t]);
 //     rs_rows_kernel<q>  one workgroup per digit scans the digit's counts over the tiles, and
 //                        leaves the digit's total (the pass adds up the totals itself: one
-//                        short launch where a scan of the whole array took two, 258 -> 222 us
+//                        short launch where a scan of the whole array took two, 259 -> 218 us
 //                        for the weighted partition of 1M atoms)
 //     rs_pass_kernel<q>  each tile ranks its keys stably by digit (eight ballots per 64
 //                        keys and per-wave running counts) and writes each digit's run
@@ -495,6 +495,17 @@ struct FilterCell {
     double c[9];
 };
 
+// The canonical d2 <= r^2.
+__device__ __forceinline__ bool filter_near(const double (&ps)[3], const double (&pt)[3], double S0, double S1,
+                                            double S2, const FilterCell& C, double r2)
+{
+    double v[3];
+    for (int a = 0; a < 3; ++a)
+        v[a] = (ps[a] - pt[a]) + fma(S2, C.c[6 + a], fma(S1, C.c[3 + a], S0 * C.c[a]));
+    const double d2 = fma(v[2], v[2], fma(v[1], v[1], v[0] * v[0]));
+    return d2 <= r2;
+}
+
 // keep iff canonical d2 <= r^2 (dist_graph_ops_kernels.cu:16-43 keeps d2 <= r2, no lower bound).
 // An edge naming an atom outside [0, n) is dropped, and raises *bad when bad is given.
 __device__ __forceinline__ bool filter_keep(const void* __restrict__ pos, int f64, int64_t n,
@@ -514,13 +525,8 @@ __device__ __forceinline__ bool filter_keep(const void* __restrict__ pos, int f6
         const float* a = (const float*)pos;
         for (int k = 0; k < 3; ++k) { ps[k] = a[3 * s + k]; pt[k] = a[3 * d + k]; }
     }
-    const double S0 = shift_at(sh, sdt, 3 * e), S1 = shift_at(sh, sdt, 3 * e + 1),
-                 S2 = shift_at(sh, sdt, 3 * e + 2);
-    double v[3];
-    for (int a = 0; a < 3; ++a)
-        v[a] = (ps[a] - pt[a]) + fma(S2, C.c[6 + a], fma(S1, C.c[3 + a], S0 * C.c[a]));
-    const double d2 = fma(v[2], v[2], fma(v[1], v[1], v[0] * v[0]));
-    return d2 <= r2;
+    return filter_near(ps, pt, shift_at(sh, sdt, 3 * e), shift_at(sh, sdt, 3 * e + 1),
+                       shift_at(sh, sdt, 3 * e + 2), C, r2);
 }
 
 __global__ void filter_flag_kernel(const void* __restrict__ pos, int f64, int64_t n, FilterCell C,
@@ -621,6 +627,193 @@ __global__ __launch_bounds__(256) void filter_write_kernel(const void* __restric
         odst[o] = d[k];
         for (int c = 0; c < 3; ++c) osh[3 * o + c] = sh[3 * (e0 + k) + c];
         ++o;
+    }
+}
+
+// ---- compaction in two passes over a mask (dg_filter_rows)
+// The targets' row of the result begins at the kept count, so a single pass cannot place it:
+// it wrote the targets to scratch, and a copy of 76 us moved them (34.5M edges, 27M kept, of
+// 735 us).  Here pass 1 leaves a bit per edge and each tile's kept count, a scan gives the
+// tiles' places, and pass 2 writes each row where it belongs; no workgroup waits for another
+// (the single pass: 641 us, its tiles numbered by tickets of 76 ns each).
+// Pass 1 (288 us) is bound by the sources' gathers: without them it takes 158 us, 6.1 TB/s;
+// half of them miss the 32 KB cache of a compute unit, atoms being in no order, and 16-byte
+// atoms gained 3 % of it, less than the pass that makes them costs.  Pass 2 (297 us) reads the
+// list again and writes the kept edges, 1.72 GB at 5.8 TB/s, the rate of plain streams here.
+// Pass 1: word i of the mask holds edges 64 i .. 64 i + 63; a wave takes kFrPer groups of 64
+// edges, their loads in flight together (with a branch for the range of the atoms before each
+// gather they wait for one another; 6 or 2 waves a SIMD in place of 4: 338, 316 us against 315).
+constexpr int kFrPer = 8;
+constexpr int kFrChunk = 64 * kFrPer;  // edges of a wave
+constexpr int kFrWaves = 8;
+constexpr int kFrTile = kFrChunk * kFrWaves;
+constexpr int kFrWords = kFrTile / 64;
+static_assert(kFrWords == 64, "a lane for each mask word of a tile");
+
+template <typename PT, typename ST>
+__global__ __launch_bounds__(64 * kFrWaves, 4) void filter_mask_kernel(
+    const PT* __restrict__ pos, int64_t na, FilterCell C, double r2, const int64_t* __restrict__ src,
+    const int64_t* __restrict__ dst, const ST* __restrict__ sh, int64_t E, uint64_t* __restrict__ mask,
+    int* __restrict__ cnt, int* __restrict__ bad)
+{
+    __shared__ int s_c[kFrWaves];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t tile = blockIdx.x;
+    const int64_t e0 = tile * kFrTile + w * kFrChunk + lane;
+    int64_t s[kFrPer], d[kFrPer];
+    ST q[kFrPer][3];
+#pragma unroll
+    for (int k = 0; k < kFrPer; ++k) {
+        const int64_t e = min(e0 + 64 * k, E - 1);
+        s[k] = src[e];
+        d[k] = dst[e];
+        for (int c = 0; c < 3; ++c) q[k][c] = sh[3 * e + c];
+    }
+    // no branch on the way to the gathers: those of several groups are in flight at a time
+    PT ps[kFrPer][3], pt[kFrPer][3];
+    bool in[kFrPer];
+#pragma unroll
+    for (int k = 0; k < kFrPer; ++k) {
+        in[k] = ((uint64_t)s[k] < (uint64_t)na) & ((uint64_t)d[k] < (uint64_t)na);
+        const int64_t a = in[k] ? s[k] : 0, b = in[k] ? d[k] : 0;
+        for (int c = 0; c < 3; ++c) {
+            ps[k][c] = pos[3 * a + c];
+            pt[k][c] = pos[3 * b + c];
+        }
+    }
+    uint64_t mine = 0;
+    int kept = 0;
+    bool out = false;
+#pragma unroll
+    for (int k = 0; k < kFrPer; ++k) {
+        const double a[3] = {(double)ps[k][0], (double)ps[k][1], (double)ps[k][2]};
+        const double b[3] = {(double)pt[k][0], (double)pt[k][1], (double)pt[k][2]};
+        const bool live = e0 + 64 * k < E;
+        const bool near = filter_near(a, b, (double)q[k][0], (double)q[k][1], (double)q[k][2], C, r2);
+        out |= live & !in[k];
+        const uint64_t m = __builtin_amdgcn_ballot_w64(live & in[k] & near);
+        mine = lane == k ? m : mine;
+        kept += __popcll(m);
+    }
+    if (out) atomicOr(bad, 1);
+    if (lane < kFrPer) mask[tile * kFrWords + w * kFrPer + lane] = mine;
+    if (lane == 0) s_c[w] = kept;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int n = 0;
+        for (int i = 0; i < kFrWaves; ++i) n += s_c[i];
+        cnt[tile] = n;
+    }
+}
+
+// A run of dwords staged in LDS at [lo, hi), to out (line aligned, the run's first dword at
+// out[lo]): 16-byte stores, whole lines but at the two ends.
+__device__ __forceinline__ void write_run(const uint32_t* buf, int lo, int hi, uint32_t* __restrict__ out, int lane)
+{
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    for (int i = 4 * lane; i < hi; i += 256) {
+        const u4 v = *(const u4*)(buf + i);
+        if (i >= lo && i + 4 <= hi) {
+            __builtin_nontemporal_store(v, (u4*)(out + i));
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (i + c >= lo && i + c < hi) out[i + c] = v[c];
+        }
+    }
+}
+
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ uint64_t readlane64(uint64_t x, int l)
+{
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, l) |
+           (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), l) << 32;
+}
+
+// Pass 2: a wave moves the kept edges of one chunk.  Their places in the tile are a scan over
+// its 64 words, a lane each.  Loads all come before stores (both count in one counter, in
+// order: a load behind a store waits for it), and the rows go through LDS, to be written in
+// 16-byte pieces of whole lines.  Non-temporal stores: the next pass over the list finds more
+// of it in the cache (pass 1 316 -> 288 us).
+constexpr int kFwWaves = 4;
+constexpr int kFwBuf = 3 * kFrChunk + 32;  // dwords: the shifts of a chunk (4-byte ones) and the skew
+
+template <typename ST>
+__global__ __launch_bounds__(64 * kFwWaves) void filter_rows_kernel(
+    const uint64_t* __restrict__ mask, const int64_t* __restrict__ off, int64_t nt,
+    const int64_t* __restrict__ src, const int64_t* __restrict__ dst, const ST* __restrict__ sh,
+    const int* __restrict__ bad, int64_t* __restrict__ out, ST* __restrict__ osh, int64_t* __restrict__ n_kept)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t s_buf[kFwWaves][kFwBuf];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t total = off[nt];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *n_kept = *bad ? -1 : total;
+    // the last tiles first: they are what the caches still hold of pass 1
+    const int64_t c = nt * kFrWaves - 1 - ((int64_t)blockIdx.x * kFwWaves + w);
+    const int64_t t = c / kFrWaves;
+    const int g0 = (int)(c % kFrWaves) * kFrPer;
+    const uint64_t m = mask[t * kFrWords + lane];
+    const int pc = __popcll(m);
+    const int ex = wave_incl_scan_dpp(pc) - pc;
+    const int x0 = __builtin_amdgcn_readlane(ex, g0);
+    const int n = __builtin_amdgcn_readlane(ex + pc, g0 + kFrPer - 1) - x0;
+    if (n == 0) return;
+    const int64_t base = off[t] + x0;
+    const int64_t e0 = c * kFrChunk + lane;
+    int64_t s[kFrPer], d[kFrPer];
+    ST q[kFrPer][3];
+    int rk[kFrPer];
+    bool keep[kFrPer];
+#pragma unroll
+    for (int k = 0; k < kFrPer; ++k) {
+        const uint64_t mk = readlane64(m, g0 + k);
+        keep[k] = mk >> lane & 1;
+        rk[k] = __builtin_amdgcn_readlane(ex, g0 + k) - x0 +
+                (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0));
+        const int64_t e = e0 + 64 * k;
+        if (keep[k]) {
+            s[k] = src[e];
+            d[k] = dst[e];
+            for (int a = 0; a < 3; ++a) q[k][a] = sh[3 * e + a];
+        }
+    }
+    uint32_t* buf = s_buf[w];
+    // skew of an address: its dwords into a line
+    auto skew = [](const void* p) { return (int)((uintptr_t)p >> 2 & 31); };
+    auto ids = [&](const int64_t (&v)[kFrPer], int64_t* o) {
+        const int lo = skew(o);
+#pragma unroll
+        for (int k = 0; k < kFrPer; ++k)
+            if (keep[k]) *(int64_t*)(buf + lo + 2 * rk[k]) = v[k];
+        wave_lds_fence();
+        write_run(buf, lo, lo + 2 * n, (uint32_t*)o - lo, lane);
+        wave_lds_fence();
+    };
+    ids(s, out + base);
+    ids(d, out + total + base);
+    // shifts: as many groups at a time as the buffer holds
+    constexpr int kDw = sizeof(ST) / 4, kParts = kDw, kGroups = kFrPer / kParts;
+#pragma unroll
+    for (int h = 0; h < kParts; ++h) {
+        const int r0 = __builtin_amdgcn_readlane(ex, g0 + h * kGroups) - x0;
+        const int r1 = h + 1 < kParts ? __builtin_amdgcn_readlane(ex, min(g0 + (h + 1) * kGroups, 63)) - x0 : n;
+        ST* o = osh + 3 * (base + r0);
+        const int lo = skew(o);
+#pragma unroll
+        for (int k = h * kGroups; k < (h + 1) * kGroups; ++k)
+            if (keep[k])
+                for (int a = 0; a < 3; ++a) *(ST*)(buf + lo + kDw * (3 * (rk[k] - r0) + a)) = q[k][a];
+        wave_lds_fence();
+        write_run(buf, lo, lo + 3 * kDw * (r1 - r0), (uint32_t*)o - lo, lane);
+        wave_lds_fence();
     }
 }
 
@@ -1013,6 +1206,75 @@ dg_status dg_filter_compact(const void* pos, int32_t pos_dtype, int64_t n_atoms,
 #undef DG_F1
     hipLaunchKernelGGL(filter_bad_kernel, dim3(1), dim3(64), 0, s, (const int*)bad, n_kept);
     return launch_ok("dg_filter_compact");
+}
+
+// Workspace of the two passes over a mask.
+struct FilterRowsLayout {
+    size_t o_cnt, o_off, o_part, o_mask, total;
+    int64_t nt;
+};
+static FilterRowsLayout filter_rows_layout(int64_t E)
+{
+    FilterRowsLayout L;
+    L.nt = (E + kFrTile - 1) / kFrTile;
+    const size_t nt = (size_t)L.nt;
+    L.o_cnt = al(8);  // behind the out-of-range flag
+    L.o_off = L.o_cnt + al(4 * (nt + 1));
+    L.o_part = L.o_off + al(8 * (nt + 1));
+    L.o_mask = L.o_part + al(8 * (nt / kScanTile + 2));
+    L.total = L.o_mask + al(8 * kFrWords * nt);
+    return L;
+}
+
+size_t dg_filter_rows_workspace_size(int64_t E)
+{
+    if (E < 0) return 0;
+    return filter_rows_layout(E).total;
+}
+
+dg_status dg_filter_rows(const void* pos, int32_t pos_dtype, int64_t n_atoms, const double* cell,
+                         double radius, const int64_t* src, const int64_t* dst, const void* shift,
+                         int32_t shift_dtype, int64_t E, int64_t* out_edges, void* out_shift,
+                         int64_t* n_kept, void* ws, size_t ws_bytes, hipStream_t s)
+{
+    dg_status st = filter_check(pos_dtype, shift_dtype, radius, E, n_atoms);
+    if (st != DG_OK) return st;
+    if (!n_kept) return fail(DG_ERR_INVALID, "n_kept is NULL");
+    const FilterRowsLayout L = filter_rows_layout(E);
+    if (ws_bytes < L.total) return fail(DG_ERR_WORKSPACE, "workspace too small");
+    if (L.nt > 0x3fffffffLL) return fail(DG_ERR_INVALID, "too many edges");
+    if (L.nt == 0) {
+        hipLaunchKernelGGL(zero_one_kernel, dim3(1), dim3(64), 0, s, n_kept);
+        return launch_ok("dg_filter_rows");
+    }
+    char* w = (char*)ws;
+    int* bad = (int*)w;
+    int* cnt = (int*)(w + L.o_cnt);
+    int64_t* off = (int64_t*)(w + L.o_off);
+    int64_t* part = (int64_t*)(w + L.o_part);
+    uint64_t* mask = (uint64_t*)(w + L.o_mask);
+    if (n_atoms == 0) pos = mask;  // every edge is out of range; an atom is loaded for it all the same
+    const FilterCell C = filter_cell(cell);
+    const double r2 = radius * radius;
+    const dim3 gm((unsigned)L.nt), gw((unsigned)(L.nt * (kFrWaves / kFwWaves)));
+    hipLaunchKernelGGL(filter_clear_kernel, dim3(1), dim3(64), 0, s, bad);
+#define DG_FM(P, T)                                                                                       \
+    hipLaunchKernelGGL((filter_mask_kernel<P, T>), gm, dim3(64 * kFrWaves), 0, s, (const P*)pos, n_atoms, \
+                       C, r2, src, dst, (const T*)shift, E, mask, cnt, bad)
+#define DG_FR(T)                                                                                          \
+    if (pos_dtype == DG_F64) DG_FM(double, T);                                                            \
+    else DG_FM(float, T);                                                                                 \
+    excl_scan<int, int64_t>(cnt, L.nt, off, part, s);                                                     \
+    hipLaunchKernelGGL(filter_rows_kernel<T>, gw, dim3(64 * kFwWaves), 0, s, (const uint64_t*)mask,       \
+                       (const int64_t*)off, L.nt, src, dst, (const T*)shift, (const int*)bad, out_edges,  \
+                       (T*)out_shift, n_kept)
+    if (shift_dtype == DG_F32) { DG_FR(float); }
+    else if (shift_dtype == DG_F64) { DG_FR(double); }
+    else if (shift_dtype == DG_I32) { DG_FR(int32_t); }
+    else { DG_FR(int64_t); }
+#undef DG_FR
+#undef DG_FM
+    return launch_ok("dg_filter_rows");
 }
 
 size_t dg_filter2_workspace_size(int64_t E)

@@ -301,23 +301,19 @@ def filter_edges_to_radius(edges, cell_shifts, pos, cell, radius):
     base = edges.data_ptr()
     with torch.cuda.device(dev):
         s = L.stream_of(dev)
-        wsb = lib.dg_filter_compact_workspace_size(E)
+        wsb = lib.dg_filter_rows_workspace_size(E)
         ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
         nk = torch.empty(1, dtype=torch.int64, device=dev)
-        # One pass: the kept edges land in order in the first k rows of E-row outputs.  The
-        # sources go straight to row 0 of the result, the targets to a scratch row, moved
-        # behind them once k is known, so edge_index is [2, k] contiguous.
+        # The kept edges land in order in the first k rows of E-row outputs, the targets right
+        # behind the k sources, so edge_index is [2, k] contiguous.
         buf = torch.empty(2 * E, dtype=torch.int64, device=dev)
-        dst_tmp = torch.empty(E, dtype=torch.int64, device=dev)
         out_s = torch.empty((E, 3), dtype=sh.dtype, device=dev)
-        L.check(lib.dg_filter_compact(L.ptr(pos), pdt, pos.size(0), cbuf, float(radius),
-                                      L.ctypes.c_void_p(base), L.ctypes.c_void_p(base + 8 * E), L.ptr(sh),
-                                      sdt, E, L.ptr(buf), L.ptr(dst_tmp), L.ptr(out_s), L.ptr(nk),
-                                      L.ptr(ws), wsb, s), "filter_edges_to_radius")
+        L.check(lib.dg_filter_rows(L.ptr(pos), pdt, pos.size(0), cbuf, float(radius),
+                                   L.ctypes.c_void_p(base), L.ctypes.c_void_p(base + 8 * E), L.ptr(sh),
+                                   sdt, E, L.ptr(buf), L.ptr(out_s), L.ptr(nk), L.ptr(ws), wsb, s),
+                "filter_edges_to_radius")
         k = int(nk.item())
         _check(k != -1, f"filter_edges_to_radius: edges hold atom indices outside [0, {pos.size(0)})")
-        _check(k >= 0, "filter_edges_to_radius: internal error (a block's wait for its predecessors gave up)")
-        buf[k:2 * k].copy_(dst_tmp[:k])
         out_e = buf[:2 * k].view(2, k)
         out_s = out_s[:k]
         if out_s.dtype != cell_shifts.dtype:

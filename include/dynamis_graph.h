@@ -216,6 +216,18 @@ dg_status dg_filter_compact(const void* pos, int32_t pos_dtype, int64_t n_atoms,
                             int64_t* out_src, int64_t* out_dst, void* out_shift, int64_t* n_kept,
                             void* workspace, size_t workspace_bytes, hipStream_t stream);
 
+/* The same filter into the edge list that filter_edges_to_radius returns: with k edges kept,
+ * out_edges[0, k) are their sources and out_edges[k, 2k) their targets, in order.  Two passes
+ * over the edge list with a bit per edge between them.
+ *   out_edges int64 [2 * n_edges] (capacity), out_shift, n_kept (-1 or the number of kept
+ *   edges) as above; workspace of dg_filter_rows_workspace_size(n_edges) bytes */
+size_t dg_filter_rows_workspace_size(int64_t n_edges);
+dg_status dg_filter_rows(const void* pos, int32_t pos_dtype, int64_t n_atoms, const double* cell,
+                         double radius, const int64_t* edge_src, const int64_t* edge_dst,
+                         const void* cell_shift, int32_t shift_dtype, int64_t n_edges,
+                         int64_t* out_edges, void* out_shift, int64_t* n_kept, void* workspace,
+                         size_t workspace_bytes, hipStream_t stream);
+
 /* SFC keys exactly as partition/sfc_kernels.cu:19-109 (curve 0 = Morton 21-bit,
  * 1 = "Hilbert" order 7), normalised by the global min / range of pos
  * (sfc_kernels.cu:196-198, range 0 -> 1).  pos fp32 [n,3]; keys int64 [n];
