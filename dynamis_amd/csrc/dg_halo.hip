@@ -45,7 +45,7 @@ enum : unsigned { kErrEdge = 1, kErrPid = 2, kErrOuter = 4 };
 
 struct Layout {
     int64_t n, W, nw, nu;
-    size_t o_hdr, o_smask, o_rflag, o_g2l, o_pid, o_hs, o_hr, o_os, o_or, o_part, total;
+    size_t o_hdr, o_smask, o_rflag, o_g2l, o_pid, o_hs, o_hr, o_os, o_or, o_part, o_loc, total;
 };
 
 Layout layout(int64_t n, int64_t W)
@@ -70,6 +70,10 @@ Layout layout(int64_t n, int64_t W)
     L.o_os = take(8 * (2 * nh + 1));
     L.o_or = L.o_os + 8 * nh;
     L.o_part = take(8 * (2 * nh / kScanTile + 2));
+    // the local atoms' bits are read by the edge pass only, before the histograms and their
+    // scan are written: in their place (one peer's are too short for them)
+    const size_t bits = al((size_t)(n + 127) / 128 * 16 + 16);
+    L.o_loc = o - L.o_hs >= bits ? L.o_hs : take(bits);
     L.total = o;
     return L;
 }
@@ -83,6 +87,7 @@ struct Args {
     int* g2l;
     uint16_t* pid16;  // pid narrowed to 16 bits (kMaxWorld <= 65535): the edge pass
                       // gathers it at random, and 2 B/atom stays in L2
+    uint64_t* local;  // bit a & 63 of word a >> 6: atom a is this rank's
 };
 
 __device__ __forceinline__ int64_t pid_at(const void* pid, int dt, int64_t a)
@@ -120,13 +125,17 @@ __global__ void clear_kernel(Args A, unsigned* hdr)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t nsm = A.n * A.nw;
+    bool mine = false;
     if (i < nsm) A.smask[i] = 0ull;
     if (i < A.n) {
         A.rflag[i] = 0;
         A.g2l[i] = -1;
         const int64_t p = pid_at(A.pid, A.pid_dt, i);
         A.pid16[i] = (uint64_t)p < (uint64_t)A.W ? (uint16_t)p : (uint16_t)0xffff;
+        mine = p == A.R;
     }
+    const uint64_t m = __builtin_amdgcn_ballot_w64(mine);
+    if ((threadIdx.x & 63) == 0 && i < A.n) A.local[i >> 6] = m;
     if (i < 16) hdr[i] = 0u;
 }
 
@@ -143,54 +152,89 @@ __global__ void g2l_kernel(Args A, const int64_t* __restrict__ outer, unsigned* 
 }
 
 // dist_graph_ops_kernels.cu:46-58 (boundary_peer_kernel) fused with the recv / send
-// marking that the reference does with unique().  A thread takes kEdgeIlp consecutive
-// edges, so that many pid gathers are in flight.  Edges of one dst arrive together, so a
+// marking that the reference does with unique().  A thread takes kEdgeIlp edges, T apart, and
+// loads the next ones before it looks at these.  Most sources are the rank's own, which one bit
+// tells; only the others' owners are gathered.  Edges of one dst arrive together, so a
 // (dst, peer) pair usually repeats on neighbouring edges: only the first edge of a run of
-// equal pairs (compared with the previous edge, across lanes too) touches the peer word.
+// equal pairs (compared with the lane before) touches the peer word.
+// Bound by the look-ups, an atom at random for each edge: gathering every source's owner took
+// 106 us for 14.4M edges of 1M atoms (2 MB of owners; the list alone is 38 us at 6 TB/s), a bit
+// of 125 KB takes 73, and 57 from LDS, where one workgroup of 1024 to a compute unit copies all
+// of them first (4 edges a thread; 8: 62, 71 without LDS).
 constexpr int kEdgeIlp = 4;
+constexpr int64_t kLocalLds = 160 << 10;  // bytes: all the LDS of a compute unit, 1.3M atoms
+// The bits go to LDS when they are more than the 32 KB that a compute unit caches anyway (100k
+// atoms, 1.4M edges: 14 us from the cache, 19 from LDS) and the edges make up for the start of
+// such workgroups, 11 us (1M atoms: 2M edges 16 / 19 us, 4M 25 / 24, 8M 43 / 37).
+constexpr int64_t kLocalCached = 32 << 10;
+constexpr int64_t kLdsEdges = 4000000;
+constexpr unsigned kCus = 256;
 
-__global__ __launch_bounds__(256) void edge_kernel(Args A, const int64_t* __restrict__ src,
-                                                   const int64_t* __restrict__ dst, int64_t E,
-                                                   unsigned* err)
+template <int T, bool LDS>
+__global__ __launch_bounds__(T) void edge_kernel(Args A, const int64_t* __restrict__ src,
+                                                 const int64_t* __restrict__ dst, int64_t E, unsigned* err)
 {
-    const int64_t e0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * kEdgeIlp;
-    int64_t s[kEdgeIlp], d[kEdgeIlp], p[kEdgeIlp];
-    bool ok[kEdgeIlp];
-#pragma unroll
-    for (int k = 0; k < kEdgeIlp; ++k) {
-        const bool in = e0 + k < E;
-        s[k] = in ? src[e0 + k] : 0;
-        d[k] = in ? dst[e0 + k] : -1;
-        ok[k] = in && (uint64_t)s[k] < (uint64_t)A.n && (uint64_t)d[k] < (uint64_t)A.n;
-        if (in && !ok[k]) atomicOr(err, (unsigned)kErrEdge);
+    __shared__ __attribute__((aligned(16))) uint32_t s_local[LDS ? kLocalLds / 4 : 4];
+    const uint32_t* const bits = (const uint32_t*)A.local;
+    if constexpr (LDS) {
+        for (int64_t i = threadIdx.x; i < (A.n + 127) / 128; i += T) ((uint4*)s_local)[i] = ((const uint4*)bits)[i];
+        __syncthreads();
     }
+    const int64_t step = (int64_t)gridDim.x * T * kEdgeIlp;
+    int64_t e0 = (int64_t)blockIdx.x * T * kEdgeIlp + threadIdx.x;
+    int64_t s[kEdgeIlp], d[kEdgeIlp], s1[kEdgeIlp], d1[kEdgeIlp];
+    auto load = [&](int64_t (&x)[kEdgeIlp], int64_t (&y)[kEdgeIlp], int64_t e) {
 #pragma unroll
-    for (int k = 0; k < kEdgeIlp; ++k) {
-        p[k] = ok[k] ? (int64_t)A.pid16[s[k]] : A.R;
-        if ((uint64_t)p[k] >= (uint64_t)A.W) {
-            atomicOr(err, (unsigned)kErrPid);
-            ok[k] = false;
-            p[k] = A.R;
+        for (int k = 0; k < kEdgeIlp; ++k) {
+            const int64_t i = min(e + T * k, E - 1);
+            x[k] = src[i];
+            y[k] = dst[i];
         }
-    }
-    // pair key of each edge (-1: nothing to mark); the previous lane's last key
-    int64_t key[kEdgeIlp];
+    };
+    load(s, d, e0);
+    for (; e0 - (int64_t)threadIdx.x < E; e0 += step) {
+        if (LDS) load(s1, d1, e0 + step);
+        bool far[kEdgeIlp];
+        unsigned any = 0;
 #pragma unroll
-    for (int k = 0; k < kEdgeIlp; ++k) key[k] = (ok[k] && p[k] != A.R) ? d[k] * A.W + p[k] : -1;
-    const unsigned lo = __shfl_up((unsigned)key[kEdgeIlp - 1], 1, 64);
-    const unsigned hi = __shfl_up((unsigned)((uint64_t)key[kEdgeIlp - 1] >> 32), 1, 64);
-    int64_t prev = (threadIdx.x & 63) ? (int64_t)(((uint64_t)hi << 32) | lo) : -1;
+        for (int k = 0; k < kEdgeIlp; ++k) {
+            const bool ok = ((uint64_t)s[k] < (uint64_t)A.n) & ((uint64_t)d[k] < (uint64_t)A.n);
+            const int64_t a = ok ? s[k] : 0;
+            const uint32_t w = LDS ? s_local[a >> 5] : bits[a >> 5];
+            const bool in = e0 + T * k < E;
+            far[k] = in & ok & !(w >> (a & 31) & 1);
+            any |= in & !ok ? (unsigned)kErrEdge : 0u;
+        }
+        if (any) atomicOr(err, any);
 #pragma unroll
-    for (int k = 0; k < kEdgeIlp; ++k) {
-        if (key[k] >= 0) {
-            A.rflag[s[k]] = 1;
-            if (key[k] != prev) {
-                unsigned long long* wp = A.smask + d[k] * A.nw + (p[k] >> 6);
-                const unsigned long long bit = 1ull << (p[k] & 63);
-                if (!(__atomic_load_n(wp, __ATOMIC_RELAXED) & bit)) atomicOr(wp, bit);
+        for (int k = 0; k < kEdgeIlp; ++k) {
+            if (__builtin_amdgcn_ballot_w64(far[k]) == 0ull) continue;
+            int64_t p = far[k] ? (int64_t)A.pid16[s[k]] : A.R;
+            if ((uint64_t)p >= (uint64_t)A.W) {
+                atomicOr(err, (unsigned)kErrPid);
+                far[k] = false;
+            }
+            // pair key of the edge (-1: nothing to mark), and the lane's before
+            const int64_t key = far[k] ? d[k] * A.W + p : -1;
+            const unsigned lo = __shfl_up((unsigned)key, 1, 64);
+            const unsigned hi = __shfl_up((unsigned)((uint64_t)key >> 32), 1, 64);
+            const int64_t prev = (threadIdx.x & 63) ? (int64_t)(((uint64_t)hi << 32) | lo) : -1;
+            if (far[k]) {
+                A.rflag[s[k]] = 1;
+                if (key != prev) {
+                    unsigned long long* wp = A.smask + d[k] * A.nw + (p >> 6);
+                    const unsigned long long bit = 1ull << (p & 63);
+                    if (!(__atomic_load_n(wp, __ATOMIC_RELAXED) & bit)) atomicOr(wp, bit);
+                }
             }
         }
-        prev = key[k];
+        if (LDS) {
+#pragma unroll
+            for (int k = 0; k < kEdgeIlp; ++k) {
+                s[k] = s1[k];
+                d[k] = d1[k];
+            }
+        }
     }
 }
 
@@ -312,6 +356,7 @@ Args make_args(const dg_halo_desc* d, const Layout& L, const void* pid, void* ws
     A.rflag = (uint8_t*)(w + L.o_rflag);
     A.g2l = (int*)(w + L.o_g2l);
     A.pid16 = (uint16_t*)(w + L.o_pid);
+    A.local = (uint64_t*)(w + L.o_loc);
     return A;
 }
 
@@ -346,9 +391,13 @@ dg_status dg_halo_count(const dg_halo_desc* d, const int64_t* src, const int64_t
     hipLaunchKernelGGL(clear_kernel, dim3(nblk(nclear)), dim3(256), 0, s, A, hdr);
     if (d->num_local > 0)
         hipLaunchKernelGGL(g2l_kernel, dim3(nblk(d->num_local)), dim3(256), 0, s, A, my_outer, err);
-    if (d->n_edges > 0)
-        hipLaunchKernelGGL(edge_kernel, dim3(nblk((d->n_edges + kEdgeIlp - 1) / kEdgeIlp)), dim3(256), 0, s, A, src, dst,
-                           d->n_edges, err);
+    const int64_t bits = (d->n_atoms + 127) / 128 * 16;
+    if (bits > kLocalCached && bits <= kLocalLds && d->n_edges >= kLdsEdges)
+        hipLaunchKernelGGL((edge_kernel<1024, true>), dim3(std::min(kCus, nblk(d->n_edges, 1024 * kEdgeIlp))),
+                           dim3(1024), 0, s, A, src, dst, d->n_edges, err);
+    else if (d->n_edges > 0)
+        hipLaunchKernelGGL((edge_kernel<256, false>), dim3(nblk(d->n_edges, 256 * kEdgeIlp)), dim3(256), 0, s, A, src,
+                           dst, d->n_edges, err);
     if (d->num_local > 0)
         hipLaunchKernelGGL(interior_kernel, dim3(nblk(d->num_local)), dim3(256), 0, s, A, my_outer,
                            interior_mask);
