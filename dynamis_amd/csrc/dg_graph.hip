@@ -2686,10 +2686,12 @@ size_t dg_graph_workspace_size(const dg_graph_desc* desc)
     return p.ws_bytes;
 }
 
-// The count stage; without slots (counts only) the sweep records no row words, and a
-// dg_graph_write that follows writes every tile from its fix-up pass instead.
+// The count stage; without words (counts only) the sweep records no row words, and a
+// dg_graph_write that follows writes every tile from its fix-up pass instead.  Without sums
+// (degrees only) the tiles' offsets and the total are not made: one launch less, 5 us of the 147
+// that the degrees of 62500 targets among 500k atoms take, of 70 in the smallest calls.
 static dg_status count_stage(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
-                             void* ws, size_t ws_bytes, int32_t* counts_out, bool slots, hipStream_t s)
+                             void* ws, size_t ws_bytes, int32_t* counts_out, bool words, bool sums, hipStream_t s)
 {
     Plan p;
     dg_status st = make_plan(desc, p);
@@ -2710,8 +2712,9 @@ static dg_status count_stage(const dg_graph_desc* desc, const void* pos, const i
         BruteArgs b = brute_args(p, pos, target_idx, ws);
         b.counts_user = counts_out;
         hipLaunchKernelGGL(brute_kernel<false>, dim3(nblocks(p.nt, 64)), dim3(64), 0, s, b);
-        excl_scan<int, int64_t>(at<int>(ws, p.o_cnt), p.nt, at<int64_t>(ws, p.o_tbase),
-                                at<int64_t>(ws, p.o_part), s, totals);
+        if (sums)
+            excl_scan<int, int64_t>(at<int>(ws, p.o_cnt), p.nt, at<int64_t>(ws, p.o_tbase),
+                                    at<int64_t>(ws, p.o_part), s, totals);
         return check_launch("dg_graph_count(brute)");
     }
     StageTimer clk(s);
@@ -2721,12 +2724,13 @@ static dg_status count_stage(const dg_graph_desc* desc, const void* pos, const i
     // 6. degrees
     SearchArgs a = search_args(p, pos, ws);
     a.counts_user = counts_out;
-    if (!slots) a.words = nullptr;
+    if (!words) a.words = nullptr;
     launch_count_kernel(a, (unsigned)p.ntiles, s);
     clk.mark("count");
     // 7. tile offsets in output order, and the total
-    excl_scan<int, int64_t>(at<int>(ws, p.o_ttot), p.ntiles, at<int64_t>(ws, p.o_tbase),
-                            at<int64_t>(ws, p.o_part), s, totals);
+    if (sums)
+        excl_scan<int, int64_t>(at<int>(ws, p.o_ttot), p.ntiles, at<int64_t>(ws, p.o_tbase),
+                                at<int64_t>(ws, p.o_part), s, totals);
     clk.mark("tile offset scan");
     st = check_launch("dg_graph_count");
     clk.report("dg_graph_count", p, -1);
@@ -2736,13 +2740,19 @@ static dg_status count_stage(const dg_graph_desc* desc, const void* pos, const i
 dg_status dg_graph_count(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
                          void* ws, size_t ws_bytes, int32_t* counts_out, hipStream_t s)
 {
-    return count_stage(desc, pos, target_idx, ws, ws_bytes, counts_out, true, s);
+    return count_stage(desc, pos, target_idx, ws, ws_bytes, counts_out, true, true, s);
 }
 
 dg_status dg_graph_counts(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
                           void* ws, size_t ws_bytes, int32_t* counts_out, hipStream_t s)
 {
-    return count_stage(desc, pos, target_idx, ws, ws_bytes, counts_out, false, s);
+    return count_stage(desc, pos, target_idx, ws, ws_bytes, counts_out, false, true, s);
+}
+
+dg_status dg_graph_degrees(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
+                           void* ws, size_t ws_bytes, int32_t* counts_out, hipStream_t s)
+{
+    return count_stage(desc, pos, target_idx, ws, ws_bytes, counts_out, false, false, s);
 }
 
 dg_status dg_graph_read_totals(const dg_graph_desc* desc, const void* ws, int64_t* total_edges,

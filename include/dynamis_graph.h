@@ -90,6 +90,11 @@ dg_status dg_graph_count(const dg_graph_desc* desc, const void* pos, const int64
 dg_status dg_graph_counts(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
                           void* workspace, size_t workspace_bytes, int32_t* counts_out,
                           hipStream_t stream);
+/* The degrees alone: dg_graph_counts without the total and the tile offsets; neither
+ * dg_graph_read_totals' total nor dg_graph_write can follow. */
+dg_status dg_graph_degrees(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
+                           void* workspace, size_t workspace_bytes, int32_t* counts_out,
+                           hipStream_t stream);
 
 /* Synchronous: copies {total_edges, flags} out of the workspace (waits for the stream).
  * Returns DG_ERR_RANGE if a data-dependent error flag is set. */
