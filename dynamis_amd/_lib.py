@@ -88,6 +88,7 @@ def lib():
         "dg_graph_degrees": (_i32, [D, _p, _p, _p, _sz, _p, _p]),
         "dg_graph_write": (_i32, [D, _p, _p, _p, _sz, _i64, _p, _p, _p, _p, _p, _i32, _p]),
         "dg_graph_write_ids": (_i32, [D, _p, _p, _p, _sz, _i64, _p, _p, _p, _p, _p, _p, _i32, _p]),
+        "dg_graph_write_n": (_i32, [D, _p, _p, _p, _sz, _i64, _p, _p, _p, _p, _p, _p, _i32, _p, _p]),
         "dg_graph_build": (_i32, [D, _p, _p, _p, _sz, _i64, _p, _p, _p, _p, _p, _p, _i32, _p]),
         "dg_graph_build_noalloc": (_i32, [D, _p, _p, _i64, _p, _p, _p, _p, _p, _p, _i32, _p, _p]),
         "dg_filter_workspace_size": (_sz, [_i64]),

@@ -718,6 +718,7 @@ struct SearchArgs {
     int64_t mapcap;
     int npools;
     int2* tmap;  // (its first entry, its entries)
+    int64_t* n_out;  // (write) where the number of edges goes too, or null
     int xsplit;     // bins ordered by x unless *xflag (see tile_sort_kernel): quarter-bin row ends
 };
 
@@ -2102,6 +2103,8 @@ __global__ __launch_bounds__(kBlock, MODE == 0 ? kCountWaves : 1) void search_ke
         search_tile<0, QS>(a, sh, blockIdx.x);
     } else {
         __shared__ FixLds f;
+        // (written here, in the build's last launch: a fill of its own took 4.5 us)
+        if (a.n_out && blockIdx.x == 0 && threadIdx.x == 0) *a.n_out = a.totals[0];
         // a grid of at most DG_FIXGRID workgroups walks the tiles: most have nothing to do,
         // and in most builds no tile has (the count pass raises totals[3] when one does)
         if (a.totals[3] == 0) return;
@@ -2184,12 +2187,14 @@ struct BruteArgs {
     int64_t capacity;
     int64_t* totals;
     const int64_t* out_ids;  // written for atom i: out_ids[i] (null: i)
+    int64_t* n_out;          // as in SearchArgs
 };
 
 template <bool WRITE>
 __global__ void brute_kernel(BruteArgs a)
 {
     int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (WRITE && a.n_out && t == 0) *a.n_out = a.totals[0];
     if (t >= a.nt) return;
     int64_t tg = a.tgt ? a.tgt[t] : t;
     if (tg < 0 || tg >= a.n) {
@@ -2787,10 +2792,10 @@ dg_status dg_graph_read_totals(const dg_graph_desc* desc, const void* ws, int64_
     return DG_OK;
 }
 
-dg_status dg_graph_write_ids(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
-                             void* ws, size_t ws_bytes, int64_t capacity, const int64_t* out_ids,
-                             int64_t* edge_src, int64_t* edge_dst, float* cell_shift, void* edge_vec,
-                             void* edge_dist, int32_t vec_dtype, hipStream_t s)
+dg_status dg_graph_write_n(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
+                           void* ws, size_t ws_bytes, int64_t capacity, const int64_t* out_ids,
+                           int64_t* edge_src, int64_t* edge_dst, float* cell_shift, void* edge_vec,
+                           void* edge_dist, int32_t vec_dtype, int64_t* n_edges, hipStream_t s)
 {
     Plan p;
     dg_status st = make_plan(desc, p);
@@ -2809,6 +2814,7 @@ dg_status dg_graph_write_ids(const dg_graph_desc* desc, const void* pos, const i
         b.out_vec = edge_vec; b.out_dist = edge_dist; b.vout_f64 = vec_dtype == DG_F64;
         b.capacity = capacity;
         b.out_ids = out_ids;
+        b.n_out = n_edges;
         hipLaunchKernelGGL(brute_kernel<true>, dim3(nblocks(p.nt, 64)), dim3(64), 0, s, b);
         return check_launch("dg_graph_write(brute)");
     }
@@ -2817,6 +2823,7 @@ dg_status dg_graph_write_ids(const dg_graph_desc* desc, const void* pos, const i
     a.out_vec = edge_vec; a.out_dist = edge_dist; a.vout_f64 = vec_dtype == DG_F64;
     a.capacity = capacity;
     a.out_ids = out_ids;
+    a.n_out = n_edges;
     if (out_ids) {
         // the ids to write in cell-list order (over the sort's scratch), so that the expansion
         // reads them from a tile's few runs
@@ -2855,6 +2862,15 @@ dg_status dg_graph_write_ids(const dg_graph_desc* desc, const void* pos, const i
     st = check_launch("dg_graph_write");
     clk.report("dg_graph_write", p, capacity);
     return st;
+}
+
+dg_status dg_graph_write_ids(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
+                             void* ws, size_t ws_bytes, int64_t capacity, const int64_t* out_ids,
+                             int64_t* edge_src, int64_t* edge_dst, float* cell_shift, void* edge_vec,
+                             void* edge_dist, int32_t vec_dtype, hipStream_t s)
+{
+    return dg_graph_write_n(desc, pos, target_idx, ws, ws_bytes, capacity, out_ids, edge_src, edge_dst,
+                            cell_shift, edge_vec, edge_dist, vec_dtype, nullptr, s);
 }
 
 dg_status dg_graph_write(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,

@@ -137,12 +137,15 @@ def build_graph(pos, cell, pbc, radius, target_indices=None, counts_only=False,
             dist = torch.empty(E, dtype=vdt, device=dev)
         if E > 0:
             src_ptr = edge_index.data_ptr()
-            L.check(lib.dg_graph_write_ids(
+            nn = torch.empty(1, dtype=torch.long, device=dev)
+            L.check(lib.dg_graph_write_n(
                 d, L.ptr(pos), L.ptr(target_indices), L.ptr(ws), wsb, E, L.ptr(out_ids),
                 L.ctypes.c_void_p(src_ptr), L.ctypes.c_void_p(src_ptr + 8 * E), L.ptr(shifts),
-                L.ptr(vec), L.ptr(dist), L.DG_F64 if vdt == torch.float64 else L.DG_F32, s),
+                L.ptr(vec), L.ptr(dist), L.DG_F64 if vdt == torch.float64 else L.DG_F32,
+                L.ptr(nn), s),
                 "radius_graph_pbc")
-        nn = torch.full((1,), E, dtype=torch.long, device=dev)
+        else:
+            nn = torch.zeros(1, dtype=torch.long, device=dev)
         out = (edge_index, shifts, nn, counts)
         if return_vectors:
             out = out + (vec, dist)

@@ -129,6 +129,13 @@ dg_status dg_graph_write_ids(const dg_graph_desc* desc, const void* pos, const i
                              const int64_t* out_ids, int64_t* edge_src, int64_t* edge_dst,
                              float* cell_shift, void* edge_vec, void* edge_dist, int32_t vec_dtype,
                              hipStream_t stream);
+/* dg_graph_write_ids that also stores the number of edges to n_edges (device, one int64; not
+ * written where there is nothing to write: no atoms or targets, or capacity 0). */
+dg_status dg_graph_write_n(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
+                           void* workspace, size_t workspace_bytes, int64_t capacity,
+                           const int64_t* out_ids, int64_t* edge_src, int64_t* edge_dst,
+                           float* cell_shift, void* edge_vec, void* edge_dist, int32_t vec_dtype,
+                           int64_t* n_edges, hipStream_t stream);
 
 /* One-call build into caller-preallocated outputs of `capacity` edges:
  * dg_graph_count then dg_graph_write, back to back on the stream with no host round trip
