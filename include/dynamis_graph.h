@@ -214,8 +214,8 @@ dg_status dg_filter_write(const void* pos, int32_t pos_dtype, int64_t n_atoms, c
 
 /* The same filter in one pass over the edge list (a decoupled look-back gives each block
  * of 4096 edges the kept count before it): kept edges go, in order, to the first n_kept
- * rows of outputs of capacity n_edges.  Replaces the same reference function; the form
- * the Python filter_edges_to_radius uses.
+ * rows of outputs of capacity n_edges, the targets in a row of their own.  Replaces the
+ * same reference function (the Python filter_edges_to_radius uses dg_filter_rows below).
  *   out_src/out_dst int64 [n_edges], out_shift [n_edges,3] of shift_dtype (capacity)
  *   n_kept  out int64 (device, one value): -1 if an edge names an atom outside
  *           [0, n_atoms), -2 if a block's wait for its predecessors gave up (a bounded wait;
