@@ -1098,7 +1098,9 @@ __device__ __forceinline__ void expand_part(const SearchArgs& a, ExpandLds<VT, G
         }
         const int64_t g0 = gb;
         gb += btot;
-        if (gb <= p0) {  // (uniform)
+        // (uniform; a batch without edges, ghosts only, names no target for a block either, and
+        // t01 would hold another batch's)
+        if (gb <= p0 || btot == 0) {
             __syncthreads();
             continue;
         }

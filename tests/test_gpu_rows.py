@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import oracle
+import plan_model
 from dynamis_amd import _lib as L
 from dynamis_amd import configs
 from dynamis_amd.dynamis_state import dynamis_state_impl as impl
@@ -15,12 +16,13 @@ from dynamis_amd.dynamis_state import dynamis_state_impl as impl
 pytestmark = pytest.mark.gpu
 
 
-def _parity(pos, cell, pbc, r, dev):
+def _parity(pos, cell, pbc, r, dev, targets=None):
+    tg = None if targets is None else torch.from_numpy(targets).to(dev)
     ei, co, _, cnt = impl.radius_graph_pbc_ex(torch.from_numpy(pos).to(dev), torch.from_numpy(cell),
-                                              torch.tensor(pbc), r, 0, False)
+                                              torch.tensor(pbc), r, 0, False, tg)
     torch.cuda.synchronize()
     used = cell.astype(pos.dtype).astype(np.float64)
-    o = oracle.radius_graph(pos, used, pbc, float(np.float32(r)))
+    o = oracle.radius_graph(pos, used, pbc, float(np.float32(r)), targets)
     assert np.array_equal(cnt.cpu().numpy(), o["counts"])
     got = oracle.canonical_sort(ei[0].cpu().numpy(), ei[1].cpu().numpy(), co.cpu().numpy().astype(np.int64))
     for a, b in zip(got, oracle.canonical_sort(o["src"], o["dst"], o["shift"])):
@@ -94,3 +96,36 @@ def test_target_ids_anywhere_in_a_line(cuda, n):
         assert torch.equal(src, src0) and torch.equal(sh, sh0)
         assert torch.equal(dst[skew:skew + E], dst0[:E])
         assert bool((dst[:skew] == -7).all()) and bool((dst[skew + E:] == -7).all())
+
+
+@pytest.mark.parametrize("seed", range(8))
+def test_batch_of_ghosts_inside_a_tile(cuda, seed):
+    """Targets 0 .. nt - 1 of a tile that holds over 512 atoms: 256 or more ghosts lie between its
+    first targets and its last, so that a batch of 256 lanes has no edges at all while the batches
+    before and behind it have.  The expansion skips it."""
+    rng = np.random.default_rng(seed)
+    r, side = 5.0, 40.0  # 15 bins an axis, tiles of 5
+    own, ghosts = [], []
+    for k in range(6):  # six tiles, none in the reach of another
+        lo, mid, hi = rng.integers(40, 250), rng.integers(520, 600), rng.integers(40, 250)
+        low = np.array([26.7 * (k & 1), 26.7 * (k >> 1 & 1), 26.7 * (k >> 2)])
+        for zlo, zhi, m, out in [(0.2, 2.5, lo, own), (2.8, 10.5, mid, ghosts), (10.8, 13.1, hi, own)]:
+            out.append(low + rng.uniform([0.1, 0.1, zlo], [13.2, 13.2, zhi], (m, 3)))
+    nt = sum(map(len, own))
+    pos = np.concatenate(own + ghosts)
+    pos[:nt] = pos[rng.permutation(nt)]
+    cell = np.eye(3) * side
+    plan = plan_model.plan(cell, (0, 0, 0), r, len(pos), nt)
+    assert plan.nb == [15] * 3 and plan.T == [5] * 3
+    # the tile's order: bin by bin, x fastest; batches of 256 with and without targets
+    b = np.minimum((pos / side * 15).astype(int), 14)
+    tile, l = (b // 5) @ [1, 3, 9], (b % 5) @ [1, 5, 25]
+    empty = 0
+    for t in np.unique(tile):
+        order = np.flatnonzero(tile == t)[np.argsort(l[tile == t], kind="stable")]
+        has = [bool((order[k:k + 256] < nt).any()) for k in range(0, len(order), 256)]
+        empty += sum(not h and any(has[:k]) and any(has[k:]) for k, h in enumerate(has))
+    assert empty > 0
+    print(f"\n[case] batch of ghosts seed={seed}: {empty} batches without edges", flush=True)
+    for dt in (np.float32, np.float64):
+        _parity(pos.astype(dt), cell, (False,) * 3, r, cuda, np.arange(nt))
