@@ -2476,8 +2476,7 @@ SearchArgs search_args(const Plan& p, const void* pos, void* ws)
     a.nrow = p.nrow;
     a.map = at<int2>(ws, p.o_map);
     a.mapcap = p.mapcap;
-    // (64 tiles or more share a pool: their sizes even out; 128 bytes each fit 8 per tile)
-    a.npools = (int)std::max<int64_t>(1, std::min<int64_t>(64, p.ntiles / 64));
+    a.npools = p.npools;  // (64 tiles or more to one: their sizes even out; 128 bytes fit 8 per tile)
     a.tmap = at<int2>(ws, p.o_wgb);  // (free once the atoms and targets are sorted)
     a.wid = a.sid;
     a.ntarg = p.nt;
@@ -2908,7 +2907,6 @@ dg_status dg_graph_build(const dg_graph_desc* desc, const void* pos, const int64
 // host-side symbol is no device address): it uses the address hipGetSymbolAddress
 // returns on each device, kept in g_scratch_ptr.
 namespace dg {
-constexpr size_t kScratchBytes = (size_t)64 << 20;
 constexpr int kMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 static std::mutex g_scratch_mu;

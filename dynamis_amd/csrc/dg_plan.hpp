@@ -30,6 +30,8 @@ constexpr int kTileMax = 6;
 constexpr int64_t kFewTiles = 1024;       // tiles below one round of workgroups on 256 CUs
 constexpr double kFewTileTargets = 192;   // expected targets per tile when tiles are few       // bins per tile along one axis
 constexpr int kCap = 1792;        // region entries staged in LDS per chunk
+constexpr int kWordsMax = 248;    // row words of a target, at most (their number is kept in a byte)
+constexpr size_t kScratchBytes = (size_t)64 << 20;  // the allocation-free build's static workspace
 
 struct Plan {
     int64_t n = 0, nt = 0;  // atoms, targets
@@ -57,10 +59,13 @@ struct Plan {
     size_t o_stmp;                   // segment-sort scratch (8 B per atom or target)
     size_t o_tkey, o_trank, o_tbcnt, o_tbstart, o_tslot, o_tsidx, o_tcaller;
     size_t o_cnt, o_ttot, o_tfix, o_tbase, o_part, o_tot, o_slot, o_nw, o_map;
-    int K = 0;              // sizes the write stage's lists: 2 K bytes per target in all
+    int K = 0;              // the write stage's lists: 2 K bytes per target at least
     int Kw = 0;             // row words per target, of those bytes
     double deg = 0;         // expected degree at the mean density
+    double words = 0;       // row words that a target may need (see plan_layout)
+    double map_even = 0, map_full = 0;  // bytes of the region map: even density, and at most
     int64_t mapcap = 0;     // region map entries: the bytes left
+    int npools = 1;         // the pools they are dealt from (64 tiles or more to a pool)
     int64_t nrow = 0;       // targets padded (group-major row length)
     size_t ws_bytes = 0;
 };
@@ -243,7 +248,7 @@ inline void plan_grid(Plan& p)
     p.band = nextafterf((float)((band + 8.0 * u * p.r2) * (1.0 + 1e-6)), INFINITY);
     p.low = nextafterf((float)((double)p.tiny * (1.0 + 1e-6) + 16.0 * u * p.r2 - (double)p.mid), INFINITY);
 
-    // Bytes per target that the write stage's lists may take (row words and region map share
+    // Bytes per target that the write stage's lists take at least (row words and region map share
     // them): from the expected degree at the mean density, with ample headroom.
     const double vol = fabs(p.C[0] * (p.C[4] * p.C[8] - p.C[5] * p.C[7]) -
                             p.C[1] * (p.C[3] * p.C[8] - p.C[5] * p.C[6]) +
@@ -254,7 +259,8 @@ inline void plan_grid(Plan& p)
     p.K = ((int)k + 7) & ~7;
 }
 
-inline void plan_layout(Plan& p)
+// lists: bytes of the row words, their counts and the region map (and o_stmp's behind them).
+inline void plan_layout_lists(Plan& p, size_t lists)
 {
     size_t o = 0;
     auto take = [&](size_t bytes) { size_t r = o; o = align_up(o + (bytes ? bytes : 1)); return r; };
@@ -296,25 +302,20 @@ inline void plan_layout(Plan& p)
     const size_t nrow = (std::max(n, nt) + 255) / 256 * 256;
     p.nrow = (int64_t)nrow;
     p.o_cnt = take(4 * nrow);
-    // 2 K bytes per target: the row words, their counts, and the region map in what is left;
-    // the map goes on over the scratch of the segment sort (tile buckets, bins of the per-bin
-    // sort: one entry per atom or target), which is free once the atoms are sorted
-    p.o_slot = take(2 * (size_t)p.K * nrow);
+    // the row words, their counts, and the region map in what is left; the map goes on over the
+    // scratch of the segment sort (tile buckets, bins of the per-bin sort: one entry per atom or
+    // target), which is free once the atoms are sorted
+    p.o_slot = take(lists);
     p.o_stmp = take(8 * std::max(n, nt));
     {
-        // The region map first: an atom is in the regions of ntl R / nb tiles per axis (on
-        // average over the bins; the tenth covers a density that favours the bins in more
-        // regions).  Then the row words: the stencil rows expected to hold an edge, with headroom
-        // for a density above the mean (a two-phase cell), and the second words of long rows (a
-        // swept row holds about twice the candidates it has edges).  A tile past the map, or a
-        // target past its words, is written by the fix-up pass.
-        double regions = 1.1 * (double)n;
-        for (int d = 0; d < 3; d++) regions *= (double)p.ntl[d] * p.R[d] / p.nb[d];
-        const double rows = std::min(4096.0, (2.0 * p.P[1] + 1.0) * (2.0 * p.P[2] + 1.0));
-        const double want = 4.0 + 1.35 * rows * (1.0 - exp(-p.deg / (0.86 * rows))) + 0.25 * p.deg;
-        const double room = ((double)(o - p.o_slot) - 8.0 * regions - (double)nrow - 1024.0) /
-                            (4.0 * (double)std::max<size_t>(nrow, 1));
-        p.Kw = (int)std::max(8.0, std::min({want, room, 248.0})) & ~3;
+        // The words that a target may need, and half of what the fullest map then leaves (unused
+        // groups and entries are never touched); where it leaves less, a map for even density.
+        auto left = [&](double map) {
+            return ((double)(o - p.o_slot) - map - (double)nrow - 1024.0) / (4.0 * (double)std::max<size_t>(nrow, 1));
+        };
+        double w = left(p.map_full);
+        w = w < p.words ? std::min(p.words, left(p.map_even)) : 0.5 * (p.words + w);
+        p.Kw = (int)std::min(std::max(w, 8.0), (double)kWordsMax) & ~3;
     }
     p.o_nw = align_up(p.o_slot + 4 * (size_t)p.Kw * nrow);
     p.o_map = align_up(p.o_nw + nrow);
@@ -326,6 +327,45 @@ inline void plan_layout(Plan& p)
     size_t big = std::max(nbins + 1, std::max(ntl, nt) + 1);
     p.o_part = take(8 * (big / 2048 + 2));
     p.ws_bytes = o;
+}
+
+inline void plan_layout(Plan& p)
+{
+    const double n = (double)p.n, nrow = (double)((std::max(p.n, p.nt) + 255) / 256 * 256);
+    const size_t least = 2 * (size_t)p.K * (size_t)nrow;
+    p.npools = (int)std::max<int64_t>(1, std::min<int64_t>(64, p.ntiles / 64));
+    // Row words per target: one for each stencil row, whatever the density around the target (a
+    // slab or a droplet fills a part of its cell only, and a list cut to the mean density sent
+    // half of its targets to the fix-up pass: 20,000 atoms in a fifth of the cell, r = 4.5, 0.26
+    // ms against 0.13), and the further words of long rows at the mean density: a row is swept over
+    // about twice the candidates it has edges, in pieces of 28 with two words each.
+    p.words = std::min(3.0 + std::min((2.0 * p.P[1] + 1.0) * (2.0 * p.P[2] + 1.0), 200.0) + 0.145 * p.deg,
+                       (double)kWordsMax);
+    // The region map has an entry for each region an atom is in: on an axis ntl R / nb of them on
+    // the average over the bins (even density; a tenth more in all), and at most those of the
+    // bin in the most regions (all atoms in such bins).  A pool may end with a tile that no
+    // longer fits it.
+    p.map_even = p.map_full = 8.8 * n;
+    for (int d = 0; d < 3; d++) {
+        const double even = (double)p.ntl[d] * p.R[d] / p.nb[d];
+        int most = 1;
+        for (int b = 0; b < p.T[d]; b++)
+            most = std::max(most, 1 + (b + p.P[d]) / p.T[d] + (p.T[d] - 1 - b + p.P[d]) / p.T[d]);
+        p.map_even *= even;
+        p.map_full *= std::max((double)most, even);
+    }
+    p.map_full = p.map_full / 1.1 * 1.05 + 8.0 * kCap * p.npools;
+    plan_layout_lists(p, least);
+    if (p.brute) return;
+    // Lists that hold this.  They never take a build out of the 64 MiB that the allocation-free
+    // build has: there they end at it.
+    const double want = 4.0 * ceil(p.words / 4.0 + 1.0) * 4.0 * nrow + nrow + p.map_full + 1024.0 -
+                        8.0 * (double)std::max(p.n, p.nt);
+    if (want <= (double)least) return;
+    const size_t base = p.ws_bytes - least;
+    size_t lists = align_up((size_t)want);
+    if (p.ws_bytes <= kScratchBytes && base + lists > kScratchBytes) lists = (kScratchBytes - base) & ~(size_t)255;
+    plan_layout_lists(p, lists);
 }
 
 }  // namespace dg

@@ -42,7 +42,8 @@ int wrap(int x, int nb, bool periodic, bool* in)
 }
 }  // namespace
 
-// out: nb[3], P[3], T[3], ntl[3], R[3], Kw, nrow, mapcap, ws_bytes, all-pairs
+// out: nb[3], P[3], T[3], ntl[3], R[3], Kw, nrow, mapcap, ws_bytes, all-pairs, ws_bytes with the
+// least lists, offset of the targets' word counts
 extern "C" int plan_numbers(const double* cell, const uint8_t* pbc, double r, int64_t n, int64_t nt, int f64,
                             int64_t* out)
 {
@@ -60,6 +61,9 @@ extern "C" int plan_numbers(const double* cell, const uint8_t* pbc, double r, in
     out[17] = p.mapcap;
     out[18] = (int64_t)p.ws_bytes;
     out[19] = p.brute;
+    out[21] = (int64_t)p.o_nw;
+    dg::plan_layout_lists(p, 2 * (size_t)p.K * (size_t)p.nrow);
+    out[20] = (int64_t)p.ws_bytes;
     return 0;
 }
 
