@@ -761,7 +761,8 @@ __device__ __forceinline__ int64_t xcd_tile_rank(int64_t b, int64_t ntiles)
 
 // LDS of one search workgroup.
 //   qbuf   the staged region: position relative to the tile centre per entry (the fix-up pass:
-//          and the atom id), with room behind it for the candidates read past a row's end;
+//          and the atom id); in the count pass with room for the three candidates read past a
+//          row's end, and before its start;
 //   rt     region bin table: the byte offset of each region bin's first entry, as 32-bit words
 //          (rp) or, with quarter-bin row ends, as four 16-bit words per bin (rq): its quarters'.
 // Positions alone (12 bytes an entry) let the count pass fit five workgroups per CU; the fix-up
@@ -775,7 +776,8 @@ static_assert(2 * kCap <= 1 << (32 - kWordBits), "a region index fits the row wo
 template <int ENT>
 struct SearchLds {
     static constexpr int kEnt = ENT;  // bytes of a region entry
-    __align__(16) unsigned char qbuf[ENT * (kCap + 3)];
+    static constexpr int kFront = ENT == 12 ? 3 * ENT : 0;  // bytes before the first one
+    __align__(16) unsigned char qbuf[kFront + ENT * (kCap + 3)];
     union {
         int tbs[kTileMax * kTileMax * kTileMax + 1];  // bin starts of the tile, while a batch's targets
                                                       // are looked up
@@ -1475,7 +1477,7 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
 {
     constexpr bool WRITE = MODE == 1;
     constexpr int kEnt = LdsOf<MODE>::type::kEnt;
-    char* const qb = (char*)sh.qbuf;
+    char* const qb = (char*)sh.qbuf + LdsOf<MODE>::type::kFront;
     int* const rp = (int*)sh.rt;
     uint16_t* const rq = (uint16_t*)sh.rt;
     TileOut out;
@@ -1822,11 +1824,12 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
             //
             // Sweeps this lane's target over the resident chunk c, in the fixed order (dz, dy, x,
             // atom) -- ascending region index.  The edge test is the sign bit of d2 - mid, shifted
-            // into a mask register, one bit per candidate and two candidates per step; a row's
+            // into a mask register, one bit per candidate and four candidates per step; a row's
             // mask becomes its row word, so the loop holds no compare, counter or store per
             // candidate.  The rare candidate within the band around the cutoff, or at a distance
             // near zero, shows in two running minima: its row is then decided again, candidate
-            // by candidate, with the exact test.
+            // by candidate, with the exact test.  (The target itself is never read: as one of the
+            // three past its piece's end, it had nearly every wave decide two pieces again.)
             //
             // Rows are swept with one row of lookahead: the wave stays on row r until every
             // lane has finished its row r, and a lane that finishes early goes on into its row
@@ -1845,8 +1848,10 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
                 int fa = 0, fe = 0;    // what is left of the row taken last
                 bool pend = false;     // some lane has some left
                 bool center = false;   // that row is the target's own
+                int lead = 0;          // candidates read before the start of the piece that ends there
                 // The next piece: at most kRowMax candidates of the row, and up to the target's own
-                // entry, which is skipped.
+                // entry, which is skipped.  The piece that ends there takes its steps up to it, so
+                // that none reads it; they start at up to three entries before the piece.
                 auto next_piece = [&]() -> int2 {
                     if (!pend) {
                         const int2 r = row_range(oz, oy, c0, c1);
@@ -1857,13 +1862,15 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
                         oz += wrap ? 1 : 0;
                         oy = wrap ? 0 : oy + 1;
                     }
-                    const int pv = fa;
+                    int pv = fa;
                     int pe = min(fe, pv + kPieceB);
                     fa = pe;
                     if (center) {
                         const bool self = vs >= pv && vs < pe;
                         pe = self ? vs : pe;
                         fa = self ? vs + kEnt : pe;
+                        lead = self ? -entries(vs - pv) & 3 : lead;
+                        pv = self ? pv - kEnt * lead : pv;
                     }
                     pend = __builtin_amdgcn_ballot_w64(fa < fe) != 0ull;
                     return make_int2(pv, pe);
@@ -1892,8 +1899,8 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
                     e = done ? pe : e;
                     while (live != 0ull) {
                         if (v < e) {
-                            // four candidates per step: those past the end (at most three, inside
-                            // qbuf) leave bits that the piece's mask drops
+                            // four candidates per step: those past the end or before the start
+                            // (at most three, inside qbuf) leave bits that the piece's mask drops
                             struct F3 { float x, y, z; };
                             const F3* const q = (const F3*)(qb + v);
                             const F3 q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
@@ -1920,17 +1927,17 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
                         v = first ? pv : nv;
                         live &= ~firstm;
                     }
-                    // the piece is done in every lane: its n candidates' bits, less
-                    // those swept past the end
-                    const int n = entries(ncur);
-                    uint32_t bits = (Mp >> (-n & 3)) & ((1u << n) - 1u);
+                    // the piece is done in every lane: its candidates' bits, less those swept past
+                    // its end or (in the piece that ends at the target) before its start
+                    const int n = entries(ncur), before = ecur == vs ? lead : 0;
+                    uint32_t bits = (Mp >> (-n & 3)) & ((1u << (n - before)) - 1u);
                     const uint64_t nearm = __builtin_amdgcn_ballot_w64(near_hi <= a.band) |
                                            __builtin_amdgcn_ballot_w64(near_lo <= a.low);
                     if (__builtin_expect((nearm | again) != 0ull, 0)) {
                         // (what the minima saw lies in this piece or, in the lookahead, the next)
                         if (__builtin_amdgcn_inverse_ballot_w64(nearm | again)) {
                             bits = 0;
-                            for (int q = ecur - ncur; q < ecur; q += kEnt) {
+                            for (int q = ecur - ncur + kEnt * before; q < ecur; q += kEnt) {
                                 const float* const x = (const float*)(qb + q);
                                 const float dx = x[0] - t0, dy = x[1] - t1, dz = x[2] - t2;
                                 const float d = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, nmid)));
