@@ -4,7 +4,7 @@
 // target's stencil rows as search_kernel<0, 1 / 2> does (lower-triangular cells: rows trimmed to
 // the cutoff, quarter-bin ends, pieces of at most 28 candidates that leave the target itself out,
 // words of 20 mask bits), in 64 bits: it counts words and region-map entries, not edges.
-#include <cstring>
+#include <utility>
 #include <vector>
 
 namespace dg {
@@ -43,7 +43,7 @@ int wrap(int x, int nb, bool periodic, bool* in)
 }  // namespace
 
 // out: nb[3], P[3], T[3], ntl[3], R[3], Kw, nrow, mapcap, ws_bytes, all-pairs, ws_bytes with the
-// least lists, offset of the targets' word counts
+// least lists, offset of the targets' word counts, pools of the map
 extern "C" int plan_numbers(const double* cell, const uint8_t* pbc, double r, int64_t n, int64_t nt, int f64,
                             int64_t* out)
 {
@@ -62,15 +62,18 @@ extern "C" int plan_numbers(const double* cell, const uint8_t* pbc, double r, in
     out[18] = (int64_t)p.ws_bytes;
     out[19] = p.brute;
     out[21] = (int64_t)p.o_nw;
+    out[22] = p.npools;
     dg::plan_layout_lists(p, 2 * (size_t)p.K * (size_t)p.nrow);
     out[20] = (int64_t)p.ws_bytes;
     return 0;
 }
 
-// Row words of every target (all atoms), words[i], and the region-map entries of all tiles.
-// pos: wrapped into the cell, [n, 3]; the cell lower-triangular with a positive diagonal.
+// Row words of every target (all atoms), words[i], and the region-map entries of all tiles: their
+// sum, and what each pool is asked for first, pools[64] (a tile asks pool ord mod npools, ord its
+// place in the output: see tile_rank_kernel, xcd_tile_rank).
+// pos: [n, 3]; the cell lower-triangular with a positive diagonal.
 extern "C" int64_t count_words(const double* cell, const uint8_t* pbc, double r, int64_t n, const double* pos,
-                               int f64, int32_t* words)
+                               int f64, int32_t* words, int64_t* pools)
 {
     Plan p;
     if (!make(p, cell, pbc, r, n, -1, f64) || p.brute) return -1;
@@ -106,6 +109,8 @@ extern "C" int64_t count_words(const double* cell, const uint8_t* pbc, double r,
     // tiles: entries of their regions, and whether the map and quarter-bin ends apply
     int64_t entries = 0;
     std::vector<int> region(p.ntiles);
+    std::vector<int64_t> asks(p.ntiles);
+    std::vector<std::pair<int64_t, int64_t>> order(p.ntiles);  // Morton code, tile
     for (int64_t t = 0; t < p.ntiles; ++t) {
         const int g[3] = {(int)(t % p.ntl[0]) * p.T[0], (int)(t / p.ntl[0] % p.ntl[1]) * p.T[1],
                           (int)(t / ((int64_t)p.ntl[0] * p.ntl[1])) * p.T[2]};
@@ -122,7 +127,22 @@ extern "C" int64_t count_words(const double* cell, const uint8_t* pbc, double r,
                 for (int x = g[0]; x < std::min(g[0] + p.T[0], nb[0]); ++x)
                     targets += (int64_t)bins[x + (size_t)nb[0] * (y + (size_t)nb[1] * z)].size();
         region[t] = (int)std::min<int64_t>(total, 1 << 30);
-        if (targets > 0 && total <= 2 * dg::kCap) entries += total;
+        asks[t] = targets > 0 && total <= 2 * dg::kCap ? total : 0;
+        entries += asks[t];
+        for (int k = 0, at = 0; k < 11; ++k)
+            for (int d = 0; d < 3; ++d)
+                if (k < p.mb[d]) {
+                    const int64_t x = d == 0 ? t % p.ntl[0] : d == 1 ? t / p.ntl[0] % p.ntl[1] : t / ((int64_t)p.ntl[0] * p.ntl[1]);
+                    order[t].first |= (x >> k & 1) << at++;
+                }
+        order[t].second = t;
+    }
+    std::sort(order.begin(), order.end());
+    constexpr int64_t kRun = 16;
+    for (int k = 0; k < 64; ++k) pools[k] = 0;
+    for (int64_t b = 0, full = p.ntiles / (8 * kRun) * (8 * kRun); b < p.ntiles; ++b) {
+        const int64_t j = b >> 3, rank = b < full ? ((j / kRun) * 8 + (b & 7)) * kRun + j % kRun : b;
+        pools[b % p.npools] += asks[order[rank].second];
     }
     const double hax = p.C[0] / nb[0], hbx = p.C[3] / nb[1], hby = p.C[4] / nb[1], hcx = p.C[6] / nb[2],
                  hcy = p.C[7] / nb[2], hcz = p.C[8] / nb[2];

@@ -1,8 +1,8 @@
 """GPU tests of the one-call build (dg_graph_build, C ABI): it must produce exactly the
 bytes of the two-stage build (dg_graph_count + dg_graph_write, itself checked against
 the oracle in test_gpu_graph.py) -- same edges in the same order, same counts -- on the
-cases that exercise every path of the fused kernel (slot expansion, targets past the slot
-capacity, chunked dense regions, explicit targets, edge vectors), and report the edge
+cases that exercise every path (the expansion, targets past their lists of row words,
+chunked dense regions, explicit targets, edge vectors), and report the edge
 count with DG_ERR_CAPACITY when the preallocated buffers are too small."""
 import numpy as np
 import pytest
@@ -50,7 +50,7 @@ def _cases():
     rng = np.random.default_rng(13)
     out.append(("dense", (rng.uniform(0, 1, (1500, 3)) * 8.0).astype(np.float32), np.eye(3) * 8.0,
                 (True, True, True), 6.0, None))
-    # a clump: targets far past the slot capacity, in a tile whose region fits LDS
+    # a clump: targets past their lists of row words, in a tile whose region fits LDS
     p = rng.uniform(0, 40.0, (6000, 3))
     p[:400] = 20.0 + rng.uniform(-1.2, 1.2, (400, 3))
     out.append(("clump", p.astype(np.float32), np.eye(3) * 40.0, (True, True, True), 5.0, None))

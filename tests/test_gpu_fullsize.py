@@ -11,7 +11,7 @@ triclinic cell scaled by 1.3934); the C5 random walk of the benchmark (degrees a
 size on frames 1, 50 and 99; every edge on a reduced box over 10 frames); and the sort
 paths no benchmark configuration reaches: more tiles than the tile-level sort takes (the
 per-bin fallback), with more than 2^24 atoms, 64-bit tile-bucket entries (more than
-2^24 targets), and a slot array past 4 GiB (64-bit slot addresses).
+2^24 targets), edge lists past 4 GiB, and row words past 4 GiB (64-bit addresses).
 """
 import itertools
 
@@ -20,6 +20,8 @@ import pytest
 import torch
 
 import oracle
+import plan_model
+from dynamis_amd import _lib as L
 from dynamis_amd import configs
 from dynamis_amd.dynamis_state import dynamis_state_impl as impl
 
@@ -207,29 +209,15 @@ def test_more_than_2_24_targets(cuda):
     assert np.array_equal(cnt.cpu().numpy(), deg[tg])
 
 
-def test_slots_past_4_gib(cuda):
-    """12M atoms at C3's density and radius (1.09e9 edges): the count pass's slot array
-    (2 bytes x 184 entries x 12M targets) is larger than 4 GiB, so slot addresses need 64
-    bits.  Checks without the oracle (whose run would take minutes here): the written edges
-    have exactly the degrees the count pass reports, each satisfies the predicate (fp64,
-    canonical form), none appears twice, and the set is symmetric under
+def _check_edges(n, box, p, ei, co):
+    """Checks without the oracle (whose run would take minutes here): every edge satisfies the
+    predicate (fp64, canonical form), none appears twice, and the set is symmetric under
     (i, j, S) <-> (j, i, -S)."""
-    n = 12_000_000
-    box = configs.uniform(n, density=0.1, seed=45, dtype=np.float32)
-    _announce(f"N={n}: slots past 4 GiB")
-    p = torch.from_numpy(box.pos).to(cuda)
-    c = torch.from_numpy(box.cell)
-    b = torch.tensor([True] * 3)
-    assert 2 * 184 * n > 2 ** 32
-    ei, co, nn, cnt = impl.radius_graph_pbc_ex(p, c, b, box.radius, 0, False)
-    E = ei.shape[1]
-    assert E > 1.0e9 and int(nn.item()) == E
-    assert torch.equal(torch.bincount(ei[1], minlength=n).to(torch.int32), cnt)
-    cell = torch.from_numpy(np.asarray(box.cell, np.float32).astype(np.float64)).to(cuda)
+    cell = torch.from_numpy(_cell_used(box)).to(p.device)
     p64 = p.double()
     r2 = float(np.float32(box.radius)) ** 2
     step = 100_000_000
-    for e0 in range(0, E, step):
+    for e0 in range(0, ei.shape[1], step):
         s_, d_ = ei[0, e0:e0 + step], ei[1, e0:e0 + step]
         v = p64[s_] + co[e0:e0 + step].double() @ cell - p64[d_]
         d2 = (v * v).sum(1)
@@ -241,3 +229,64 @@ def test_slots_past_4_gib(cuda):
     assert bool((fwd[1:] > fwd[:-1]).all())  # no edge twice
     rev = torch.sort(_keys_torch(ei[1], ei[0], -S, nb, sb)).values
     assert torch.equal(fwd, rev)
+
+
+def test_slots_past_4_gib(cuda):
+    """12M atoms at C3's density and radius: 1.09e9 edges, so each of the outputs is past 4 GiB
+    (8.7 to 13 GB) and edges' addresses need 64 bits; the written edges have exactly the degrees
+    that the count pass reports."""
+    n = 12_000_000
+    box = configs.uniform(n, density=0.1, seed=45, dtype=np.float32)
+    _announce(f"N={n}: edge lists past 4 GiB")
+    p = torch.from_numpy(box.pos).to(cuda)
+    c = torch.from_numpy(box.cell)
+    b = torch.tensor([True] * 3)
+    ei, co, nn, cnt = impl.radius_graph_pbc_ex(p, c, b, box.radius, 0, False)
+    E = ei.shape[1]
+    assert E > 1.0e9 and int(nn.item()) == E
+    assert 8 * E > 2 ** 32
+    assert torch.equal(torch.bincount(ei[1], minlength=n).to(torch.int32), cnt)
+    _check_edges(n, box, p, ei, co)
+
+
+def test_row_words_past_4_gib(cuda):
+    """44M atoms, sparse but for 200 dense clumps whose targets fill their lists of row words: a
+    target's groups of four words lie a row of the array apart (16 bytes a target), so the last
+    ones of a list are past 4 GiB, and a 32-bit address would fall into the first groups of others.
+    Which groups were written is read from the workspace."""
+    n, r, side = 44_000_000, 5.0, 1664.0  # 5 neighbours a target on the average
+    rng = np.random.default_rng(46)
+    pos = rng.uniform(0.0, side, (n, 3)).astype(np.float32)
+    at = 0
+    for k in range(200):
+        m = int(rng.integers(100, 700))
+        d = rng.normal(size=(m, 3))
+        d *= (5.0 * rng.uniform(0.0, 1.0, m) ** (1.0 / 3.0) / np.linalg.norm(d, axis=1))[:, None]
+        pos[at:at + m] = rng.uniform(10.0, side - 10.0, 3) + d
+        at += m
+    box = configs.Box("clumps", pos, np.eye(3) * side, (True, True, True), r)
+    _announce(f"N={n}: row words past 4 GiB")
+    lib = L.lib()
+    p, c = torch.from_numpy(pos).to(cuda), torch.from_numpy(box.cell)
+    d = impl._desc(p, c, torch.tensor([True] * 3), impl._r32(r), None)
+    plan = plan_model.plan(box.cell, box.pbc, impl._r32(r), n)
+    wsb = lib.dg_graph_workspace_size(d)
+    assert plan.ws_bytes == wsb
+    ws = torch.zeros(wsb, dtype=torch.uint8, device=cuda)
+    cnt = torch.empty(n, dtype=torch.int32, device=cuda)
+    s = L.stream_of(cuda)
+    L.check(lib.dg_graph_count(d, L.ptr(p), None, L.ptr(ws), wsb, L.ptr(cnt), s), "dg_graph_count")
+    tot, flags = L._i64(0), L._i64(0)
+    L.check(lib.dg_graph_read_totals(d, L.ptr(ws), tot, flags, s), "totals")
+    E = int(tot.value)
+    words = ws[plan.o_nw:plan.o_nw + n].to(torch.int64)
+    last = torch.where(words <= plan.Kw, (words - 1) // 4, 0) * 16 * plan.nrow  # (255: past the list)
+    assert int((last > 2 ** 32).sum()) > 100
+    del words, last
+    ei = torch.empty((2, E), dtype=torch.int64, device=cuda)
+    co = torch.empty((E, 3), dtype=torch.float32, device=cuda)
+    base = ei.data_ptr()
+    L.check(lib.dg_graph_write(d, L.ptr(p), None, L.ptr(ws), wsb, E, L.ctypes.c_void_p(base),
+                               L.ctypes.c_void_p(base + 8 * E), L.ptr(co), None, None, L.DG_F32, s), "dg_graph_write")
+    assert torch.equal(torch.bincount(ei[1], minlength=n).to(torch.int32), cnt)
+    _check_edges(n, box, p, ei, co)

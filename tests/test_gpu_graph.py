@@ -339,8 +339,8 @@ def _two_phase_box():
 @pytest.mark.parametrize("which", ["c4", "two-phase"])
 def test_edge_vectors(cuda, which):
     """Edge vectors and distances (fp64 bit-identical to the canonical formula, fp32 the
-    correctly rounded values); the two-phase box has two-chunk tiles, whose edges come from
-    the fix-up kernel's expansion."""
+    correctly rounded values); the two-phase box has two-chunk tiles, whose region map is longer
+    than the expansion's LDS holds."""
     box = configs.c4(scale=0.4) if which == "c4" else _two_phase_box()
     r = box.radius
     o = oracle.radius_graph(box.pos, box.cell, box.pbc, r, vectors=True)
@@ -527,9 +527,8 @@ def test_near_cutoff_pairs_along_x(cuda, dtype, shape):
 @pytest.mark.parametrize("shape", ["cubic", "lowtri"])
 def test_crowded_bins_in_sparse_rows(cuda, shape):
     """Bins of 16 to 80 atoms (spread over the whole bin) in a background at C3's density,
-    each tile still one LDS chunk: the count's quarter-bin prefix counts saturate at 15 in
-    these bins, and rows that start or end in them must fall back to the whole bin on the
-    saturated side."""
+    each tile still one LDS chunk: the count's quarter-bin row ends inside bins that hold many
+    atoms, and rows of more candidates than one word or one sweep piece."""
     cell = {"cubic": np.eye(3) * 45.0,
             "lowtri": np.array([[45.0, 0, 0], [10.0, 44.0, 0], [-6.0, 8.0, 43.0]])}[shape]
     r = 6.0
@@ -586,9 +585,8 @@ def _two_phase(side, rho_lo, rho_hi, seed):
 @pytest.mark.parametrize("side,rho_lo,rho_hi,r", [(60.0, 0.2, 0.02, 6.0), (50.0, 0.3, 0.01, 5.0)])
 def test_two_phase_dense_tiles(cuda, side, rho_lo, rho_hi, r):
     """A two-phase box: tiles are planned for the mean density, so in the dense phase the
-    region needs two LDS chunks (slots over both chunks, expanded by the fix-up kernel) and
-    many targets exceed the slot capacity (their edges k >= K swept again across both
-    chunks)."""
+    region needs two LDS chunks (row words and a region map over both), and the tiles' targets
+    go in several batches."""
     pos, cell = _two_phase(side, rho_lo, rho_hi, 5)
     check_parity(pos, cell, (1, 1, 1), r, cuda, name=f"two-phase {side} {rho_lo}/{rho_hi}")
 
@@ -596,10 +594,10 @@ def test_two_phase_dense_tiles(cuda, side, rho_lo, rho_hi, r):
 @pytest.mark.parametrize("side,cube,rho_bg,rho_c", [(60.0, 24.0, 0.005, 0.5), (64.0, 26.0, 0.004, 0.45)])
 def test_dense_cube_in_sparse_box(cuda, side, cube, rho_bg, rho_c):
     """A dense cube in a sparse periodic box, r = 5: tiles are planned for the mean
-    density, so around the cube regions need two, three or four LDS chunks, and the cube's
-    targets have several times the slot capacity K.  Covers every fix-up path: targets past
-    K in one- and two-chunk regions (slots, then a second sweep across the chunks) and in
-    regions of more than two chunks (written directly, chunk by chunk)."""
+    density, so around the cube regions need two, three or four LDS chunks, and many of the
+    cube's targets have more row words than their lists hold.  Covers every fix-up path: such
+    targets in one- and two-chunk regions (swept again across the chunks) and regions of more
+    than two chunks (written directly, chunk by chunk)."""
     rng = np.random.default_rng(11)
     bg = rng.uniform(0, side, (int(rho_bg * side ** 3), 3))
     cl = rng.uniform(0, cube, (int(rho_c * cube ** 3), 3)) + (side - cube) / 2

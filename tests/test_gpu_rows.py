@@ -63,6 +63,21 @@ def test_close_pairs(cuda, dtype):
     _parity(pos, np.eye(3) * 24.0, (True, True, True), 5.0, cuda)
 
 
+def _vectors_agree(pos, cell, r, dev):
+    """The build with vectors and distances: the same edges, and their vectors in 64 bits."""
+    p, c, b = torch.from_numpy(pos).to(dev), torch.from_numpy(cell), torch.tensor([True] * 3)
+    ei, co, _, cnt = impl.radius_graph_pbc_ex(p, c, b, r, 0, False)
+    ei2, co2, _, cnt2, vec, dist = impl.radius_graph_pbc_vectors(p, c, b, r)
+    assert torch.equal(ei2, ei) and torch.equal(co2, co) and torch.equal(cnt2, cnt)
+    used = c.to(p.dtype).double().to(dev)
+    v = p.double()[ei[0]] - p.double()[ei[1]] + co.double() @ used
+    # (a vector is a 64-bit result: three products and sums of at most 400 A, rounded once more
+    # where the outputs are 32-bit)
+    tol = 400 * 2.0 ** -50 + (5.0 * 2.0 ** -24 if vec.dtype == torch.float32 else 0.0)
+    assert float((vec.double() - v).abs().max()) <= tol
+    assert float((dist.double() - v.norm(dim=1)).abs().max()) <= 2 * tol
+
+
 def _build(pos, cell, dev, r, cap, skew):
     """dg_graph_build with the target ids `skew` entries into an array that starts on a line, and
     guard values around every output."""
@@ -129,3 +144,47 @@ def test_batch_of_ghosts_inside_a_tile(cuda, seed):
     print(f"\n[case] batch of ghosts seed={seed}: {empty} batches without edges", flush=True)
     for dt in (np.float32, np.float64):
         _parity(pos.astype(dt), cell, (False,) * 3, r, cuda, np.arange(nt))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("spill,xs", [("one pool full", (5, 6)), ("all pools full", (4, 6))])
+def test_region_map_spills(cuda, spill, xs, dtype):
+    """A column of atoms along z, in every other stretch of 20 bins of 156 and in those bins along x
+    and y that most tiles' regions hold: all tiles ask one of the map's two pools, which has not
+    the room.  The others' entries go to the second pool, or, where that fills too, their tiles to
+    the fix-up pass; the edges and their vectors are the same."""
+    n, r, cell = 2400, 5.0, np.diag([15.6, 15.6, 391.5])  # 6 x 6 x 156 bins
+    rng = np.random.default_rng(1)
+    f = rng.uniform(0.0, 1.0, (n, 3))
+    f[:, 0] = (xs[0] + f[:, 0] * (xs[1] - xs[0])) / 6
+    f[:, 1] = (4 + 2 * f[:, 1]) / 6
+    f[:, 2] = (40 * rng.integers(0, 4, n) + 20 * f[:, 2]) / 156
+    pos = (f @ cell).astype(dtype)
+    plan = plan_model.plan(cell, (1, 1, 1), r, n, f64=dtype is np.float64)
+    words, pools = plan_model.row_words(pos, cell, (1, 1, 1), r)
+    assert plan.npools == 2 and words.max() <= plan.Kw  # (no target goes to the fix-up pass by itself)
+    assert pools[0] > 1.1 * plan.mapcap / 2 and pools[1] == 0
+    assert pools[0] > 1.1 * plan.mapcap if spill == "all pools full" else pools[0] < 0.9 * plan.mapcap
+    print(f"\n[case] region map, {spill} {np.dtype(dtype)}", flush=True)
+    _parity(pos, cell, (True,) * 3, r, cuda)
+    _vectors_agree(pos, cell, r, cuda)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("shape", ["cubic", "sheared"])
+def test_targets_past_their_list(cuda, shape, dtype):
+    """A dense clump in an even box: its targets have more row words than their lists hold and go
+    to the fix-up pass, in tiles whose other targets the expansion writes."""
+    rng = np.random.default_rng(13)
+    pos = rng.uniform(0.0, 40.0, (6000, 3))
+    pos[:400] = 20.0 + rng.uniform(-1.2, 1.2, (400, 3))
+    cell = np.eye(3) * 40.0
+    if shape == "sheared":
+        cell[1, 0], cell[2, 0], cell[2, 1] = 6.0, -4.0, 5.0
+    pos, r = pos.astype(dtype), 5.0
+    plan = plan_model.plan(cell, (1, 1, 1), r, len(pos), f64=dtype is np.float64)
+    words, _ = plan_model.row_words(pos, cell, (1, 1, 1), r)
+    assert 100 < int((words > plan.Kw).sum()) < 1000
+    print(f"\n[case] targets past their list {shape} {np.dtype(dtype)}", flush=True)
+    _parity(pos, cell, (True,) * 3, r, cuda)
+    _vectors_agree(pos, cell, r, cuda)

@@ -42,11 +42,11 @@ CASES = (
 def test_lists_hold_every_target(name, make, args, r):
     pos, cell = make(*args)
     plan = plan_model.plan(cell, (1, 1, 1), r, len(pos))
-    words, entries = plan_model.row_words(pos, cell, (1, 1, 1), r)
+    words, pools = plan_model.row_words(pos, cell, (1, 1, 1), r)
     assert words.max() > 0
     # (the fullest list of 20,000 leaves a fifth: no structure of its kind is near the end)
     assert words.max() <= 0.8 * plan.Kw
-    assert entries <= 0.96 * plan.mapcap
+    assert pools.sum() <= 0.96 * plan.mapcap
 
 
 @pytest.mark.parametrize("r,rho", [(4.5, 0.02), (5.0, 0.05), (6.0, 0.1), (10.0, 0.1)])
