@@ -55,14 +55,15 @@ def _batch_in_one_pass(natoms, cells=None, pbc=(True, True, True), radius=6.0) -
     ``cells`` every structure is costed at the measured image count."""
     if len(natoms) < 2 or max(natoms) > BATCH_MAX_ATOMS:
         return False
-    if cells is None:
-        weights = 1.0
-    else:
+    if cells is not None:
         images = _images_per_pair(np.asarray(cells, dtype=np.float64).reshape(-1, 3, 3), pbc, radius)
         if images.max() > BATCH_MAX_IMAGES:
             return False
         weights = images / _BATCH_IMAGES_MEASURED
-    pairs = float((np.asarray(natoms, dtype=np.float64) ** 2 * weights).sum())
+    pairs = np.asarray(natoms, dtype=np.float64) ** 2
+    if cells is not None:  # (cells past the structures, as a padded batch has them, cost nothing)
+        pairs = pairs[:len(weights)] * weights[:len(pairs)]
+    pairs = float(pairs.sum())
     return _BATCH_MS + _BATCH_MS_PER_PAIR * pairs < _LOOP_MS_PER_STRUCTURE * len(natoms)
 
 

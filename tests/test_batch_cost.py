@@ -34,3 +34,13 @@ def test_images_of_a_batch(pbc):
     # a handful of roundings in 64 bits each (determinants of random cells lose a few digits)
     np.testing.assert_allclose(got[fin], want[fin], rtol=1e-10)
     assert wrap._images_per_pair(cells[0], pbc, 6.0) == pytest.approx(want[0], rel=1e-10)
+
+
+@pytest.mark.parametrize("natoms", [[10, 10], [8000, 8000], [250] * 128])
+def test_cells_of_a_padded_batch(natoms):
+    """More cells than structures: the first ones count, as in the loop over the structures."""
+    cells = np.repeat(np.eye(3)[None] * 46.0, len(natoms), axis=0)
+    want = wrap._batch_in_one_pass(natoms, cells, [True] * 3, 6.0)
+    for more in (1, 3):
+        padded = np.concatenate([cells, np.eye(3)[None].repeat(more, axis=0) * 30.0])
+        assert wrap._batch_in_one_pass(natoms, padded, [True] * 3, 6.0) == want
