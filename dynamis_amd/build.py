@@ -19,9 +19,7 @@ SOURCES = ["dg_graph.hip", "dg_count.hip", "dg_sfc.hip", "dg_halo.hip", "dg_batc
 # Per-source flags.  The count kernel's sweep is bound by VALU issue: LLVM's iterative ILP
 # scheduler orders it better (1M atoms: 282 -> 271 us), while the default scheduler
 # suits the store-bound write kernels of dg_graph.hip (0.660 vs 0.671 ms under ILP).
-# The halo plan's edge pass is alike under both (62 us for 14.4M edges).
-SOURCE_FLAGS = {"dg_count.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
-                "dg_halo.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]}
+SOURCE_FLAGS = {"dg_count.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]}
 ARCH = os.environ.get("DG_OFFLOAD_ARCH", "gfx950")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
