@@ -15,11 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libdynamis_graph.so")
-SOURCES = ["dg_graph.hip", "dg_count.hip", "dg_sfc.hip", "dg_halo.hip", "dg_batch.hip"]
-# Per-source flags.  The count kernel's sweep is bound by VALU issue: LLVM's iterative ILP
-# scheduler orders it better (1M atoms: 282 -> 271 us), while the default scheduler
-# suits the store-bound write kernels of dg_graph.hip (0.660 vs 0.671 ms under ILP).
-SOURCE_FLAGS = {"dg_count.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]}
+SOURCES = ["dg_graph.hip", "dg_sfc.hip", "dg_halo.hip", "dg_batch.hip"]
 ARCH = os.environ.get("DG_OFFLOAD_ARCH", "gfx950")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -50,7 +46,7 @@ def build(verbose: bool = False) -> str:
     os.makedirs(bdir, exist_ok=True)
     for src in SOURCES:
         obj = os.path.join(bdir, src.replace(".hip", ".o"))
-        out = _run([HIPCC, *FLAGS, *SOURCE_FLAGS.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj])
+        out = _run([HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj])
         if verbose and out.strip():
             print(out)
         objs.append(obj)

@@ -38,19 +38,8 @@
 #include "dg_scan.hpp"
 #include "dg_segsort.hpp"
 
-// The count kernel (search_kernel<0>) is compiled in a translation unit of its own,
-// dg_count.hip, which includes this file with DG_COUNT_TU defined: there, only the
-// device code the count kernel needs and its launcher are compiled (under another
-// instruction-scheduling strategy, see build.py), and everything else is left out.
-#ifdef DG_COUNT_TU
-#define DG_MAIN_TU 0
-#else
-#define DG_MAIN_TU 1
-#endif
-
 namespace dg {
 
-#if DG_MAIN_TU
 thread_local std::string g_last_error;
 
 dg_status fail(dg_status st, const std::string& msg)
@@ -58,7 +47,6 @@ dg_status fail(dg_status st, const std::string& msg)
     g_last_error = msg;
     return st;
 }
-#endif
 
 constexpr int kRegPerThread = (kMaxRegion + kBlock - 1) / kBlock;
 constexpr int kBinSortMax = 128;
@@ -115,7 +103,6 @@ __device__ __forceinline__ float bin_xkey(const float4& e, const XKey& k)
     return fmaf(-fc, k.hcx, fmaf(-fb, k.hbx, e.x));
 }
 
-#if DG_MAIN_TU
 // ---------------------------------------------------------------- tile SFC ranks
 // Rank of every tile in the compact Morton order (morton_encode) among the tiles of the
 // grid, computed directly: for each 1 bit of the tile's code, the tiles whose codes share
@@ -635,8 +622,6 @@ __global__ void finish_targets_kernel(int64_t nbins, int64_t n, const int* __res
         tsidx[j] = inv[a];
     }
 }
-
-#endif  // DG_MAIN_TU (sort kernels)
 
 // ---------------------------------------------------------------- neighbour search
 struct SearchArgs {
@@ -1815,12 +1800,13 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
                 put_word(((uint32_t)last << kWordBits) | bits, bits != 0u);
             };
 
-            // Bound by VALU issue and, per row, by the latency of its few LDS reads: 120M VALU
-            // instructions at 1M atoms (r = 6, 90.5M edges) in 0.27 ms, against 159M in 0.345 ms
+            // Bound by VALU issue and, per row, by the latency of its few LDS reads: 113M VALU
+            // instructions at 1M atoms (r = 6, 90.5M edges) in 0.257 ms, against 159M in 0.345 ms
             // for a sweep that wrote a 2-byte entry per edge (two candidates a step, 34 VALU;
             // this one: four a step, 39), at four workgroups per CU to this one's five.
-            // Where a row holds three candidates the width gains nothing and one tile's chain of
-            // rows is longer: 42 against 36 us for 20000 atoms of 0.05 per cubic A, r = 4.5.
+            // Where a row holds three candidates the width gains nothing: 35 against 33 us for the
+            // degrees of 20000 atoms of 0.05 per cubic A, r = 4.5; 41 against 37 with the row words
+            // and the region map, which take 5 us off the expansion.
             //
             // Sweeps this lane's target over the resident chunk c, in the fixed order (dz, dy, x,
             // atom) -- ascending region index.  The edge test is the sign bit of d2 - mid, shifted
@@ -1829,7 +1815,8 @@ __device__ __forceinline__ TileOut search_tile(const SearchArgs& a,
             // candidate.  The rare candidate within the band around the cutoff, or at a distance
             // near zero, shows in two running minima: its row is then decided again, candidate
             // by candidate, with the exact test.  (The target itself is never read: as one of the
-            // three past its piece's end, it had nearly every wave decide two pieces again.)
+            // three past its piece's end, it had nearly every wave decide two pieces again, 121M
+            // VALU instructions and 24 us more.)
             //
             // Rows are swept with one row of lookahead: the wave stays on row r until every
             // lane has finished its row r, and a lane that finishes early goes on into its row
@@ -2126,10 +2113,6 @@ __global__ __launch_bounds__(kBlock, MODE == 0 ? kCountWaves : 1) void search_ke
         }
     }
 }
-
-#if DG_MAIN_TU
-// the count kernel's launcher, compiled in dg_count.hip
-void launch_count_kernel(const SearchArgs& a, unsigned grid, hipStream_t s);
 
 // The positions in cell-list order (entry g: atom sid[g]), for the edge vectors: the
 // expansion then reads a tile's sources from a few contiguous runs instead of from all
@@ -2671,7 +2654,6 @@ void launch_sort(const Plan& p, const void* pos, const int64_t* target_idx, void
     }
 }
 
-#else   // DG_COUNT_TU
 void launch_count_kernel(const SearchArgs& a, unsigned grid, hipStream_t s)
 {
     if (a.lowtri == 2 && a.xsplit)
@@ -2681,13 +2663,11 @@ void launch_count_kernel(const SearchArgs& a, unsigned grid, hipStream_t s)
     else
         hipLaunchKernelGGL((search_kernel<0, 0>), dim3(grid), dim3(kBlock), 0, s, a);
 }
-#endif  // DG_MAIN_TU
 
 }  // namespace dg
 
 using namespace dg;
 
-#if DG_MAIN_TU
 extern "C" {
 
 const char* dg_last_error(void) { return g_last_error.c_str(); }
@@ -2703,8 +2683,8 @@ size_t dg_graph_workspace_size(const dg_graph_desc* desc)
 
 // The count stage; without words (counts only) the sweep records no row words, and a
 // dg_graph_write that follows writes every tile from its fix-up pass instead.  Without sums
-// (degrees only) the tiles' offsets and the total are not made: one launch less, 5 us of the 147
-// that the degrees of 62500 targets among 500k atoms take, of 70 in the smallest calls.
+// (degrees only) the tiles' offsets and the total are not made: one launch less, 5 us where the
+// degrees of 62500 targets among 500k atoms take 124, those of the smallest boxes 98.
 static dg_status count_stage(const dg_graph_desc* desc, const void* pos, const int64_t* target_idx,
                              void* ws, size_t ws_bytes, int32_t* counts_out, bool words, bool sums, hipStream_t s)
 {
@@ -3038,4 +3018,3 @@ extern "C" dg_status dg_graph_build_noalloc(const dg_graph_desc* desc, const voi
     }
     return rs;
 }
-#endif  // DG_MAIN_TU

@@ -30,7 +30,6 @@ def test_host_code_under_asan_ubsan():
         objs = []
         for src in b.SOURCES:
             obj = os.path.join(d, src + ".o")
-            # (the per-source scheduler flags are left out: device code is not run here)
             cmd = [b.HIPCC, *flags, "-c", os.path.join(b.CSRC, src), "-o", obj]
             r = subprocess.run(cmd, capture_output=True, text=True)
             assert r.returncode == 0, r.stdout + r.stderr
