@@ -159,8 +159,8 @@ __global__ void g2l_kernel(Args A, const int64_t* __restrict__ outer, unsigned* 
 // equal pairs (compared with the lane before) touches the peer word.
 // Bound by the look-ups, an atom at random for each edge: gathering every source's owner took
 // 106 us for 14.4M edges of 1M atoms (2 MB of owners; the list alone is 38 us at 6 TB/s), a bit
-// of 125 KB takes 73, and 57 from LDS, where one workgroup of 1024 to a compute unit copies all
-// of them first (4 edges a thread; 8: 62, 71 without LDS).
+// of 125 KB takes 73, and 57 from LDS (60 inside the whole plan), where one workgroup of 1024 to a
+// compute unit copies all of them first (4 edges a thread; 8: 62, 71 without LDS).
 constexpr int kEdgeIlp = 4;
 constexpr int64_t kLocalLds = 160 << 10;  // bytes: all the LDS of a compute unit, 1.3M atoms
 // The bits go to LDS when they are more than the 32 KB that a compute unit caches anyway (100k
