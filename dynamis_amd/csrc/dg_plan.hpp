@@ -358,13 +358,15 @@ inline void plan_layout(Plan& p)
     plan_layout_lists(p, least);
     if (p.brute) return;
     // Lists that hold this.  They never take a build out of the 64 MiB that the allocation-free
-    // build has: there they end at it.
+    // build has, nor past 64 GiB (a quarter of the card: 270M sparse atoms): there they end.
     const double want = 4.0 * ceil(p.words / 4.0 + 1.0) * 4.0 * nrow + nrow + p.map_full + 1024.0 -
                         8.0 * (double)std::max(p.n, p.nt);
     if (want <= (double)least) return;
     const size_t base = p.ws_bytes - least;
     size_t lists = align_up((size_t)want);
-    if (p.ws_bytes <= kScratchBytes && base + lists > kScratchBytes) lists = (kScratchBytes - base) & ~(size_t)255;
+    for (size_t end : {kScratchBytes, kScratchBytes << 10})
+        if (p.ws_bytes <= end && base + lists > end) lists = (end - base) & ~(size_t)255;
+    if (base + lists > kScratchBytes << 10) lists = least;
     plan_layout_lists(p, lists);
 }
 

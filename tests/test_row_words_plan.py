@@ -53,9 +53,22 @@ def test_lists_hold_every_target(name, make, args, r):
 def test_the_lists_end_at_the_static_workspace(r, rho):
     """No build leaves the 64 MiB of the allocation-free build for its lists: past the atoms where
     the workspace reaches it, it stays there until the least lists need more."""
-    limit = 64 << 20
+    _ends_at(64 << 20, 2e4, 6e5, r, rho)
+
+
+@pytest.mark.parametrize("r,rho", [(4.5, 0.02), (5.0, 0.05)])
+def test_the_lists_of_the_largest_builds(r, rho):
+    """Nor do they take a build past 64 GiB, and one that is past it has the least lists: what fitted
+    the card before still does."""
+    _ends_at(64 << 30, 1e8, 4e8, r, rho)
+    n = 500_000_000
+    plan = plan_model.plan(np.eye(3) * (n / rho) ** (1.0 / 3.0), (1, 1, 1), r, n)
+    assert plan.ws_bytes == plan.least_bytes > 64 << 30
+
+
+def _ends_at(limit, lo, hi, r, rho):
     sizes = []
-    for n in np.unique(np.geomspace(2e4, 6e5, 400).astype(int)):
+    for n in np.unique(np.geomspace(lo, hi, 400).astype(int)):
         cell = np.eye(3) * (n / rho) ** (1.0 / 3.0)
         sizes.append((n, plan_model.plan(cell, (1, 1, 1), r, int(n)).ws_bytes))
     below = [s for _, s in sizes if s <= limit]
